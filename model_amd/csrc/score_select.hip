@@ -121,20 +121,18 @@ __device__ __forceinline__ W& lds_at(W* arr, uint32_t byte_off) {
 // partner lane's arrives through v_permlane32_swap): the element-wise max of
 // the own list and the partner's reversed list is the union's top KMAX as a
 // bitonic sequence, so its minimum is the KMAX-th largest.  Both lanes of the
-// pair get the same key; 0 when the union holds fewer than KMAX keys.
+// pair get the same key; kNoKey when the union holds fewer than KMAX keys.
 template <int KMAX, bool NOISE>
-__device__ __forceinline__ u64 pair_kth_key(const TopList<KMAX, NOISE>& top, int par) {
-  u64 m = ~0ull;
+__device__ __forceinline__ Key pair_kth_key(const TopList<KMAX, NOISE>& top, int par) {
+  Key m = __builtin_bit_cast(Key, 0x7FEFFFFFFFFFFFFFull);  // above every key
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
-    float lo = __uint_as_float((uint32_t)top.key[j]), lo2 = lo;
-    float hi = __uint_as_float((uint32_t)(top.key[j] >> 32)), hi2 = hi;
+    float lo = __uint_as_float(key_lo(top.key[j])), lo2 = lo;
+    float hi = __uint_as_float(key_hi(top.key[j])), hi2 = hi;
     half_swap(lo, lo2);
     half_swap(hi, hi2);
-    const u64 other = ((u64)__float_as_uint(par ? hi : hi2) << 32) | __float_as_uint(par ? lo : lo2);
-    const u64 own = top.key[KMAX - 1 - j];
-    const u64 c = own > other ? own : other;
-    m = c < m ? c : m;
+    const Key other = key_of(__float_as_uint(par ? hi : hi2), __float_as_uint(par ? lo : lo2));
+    m = __builtin_fmin(m, __builtin_fmax(top.key[KMAX - 1 - j], other));
   }
   return m;
 }
@@ -147,15 +145,15 @@ __device__ __forceinline__ u64 pair_kth_key(const TopList<KMAX, NOISE>& top, int
 // past the lane's count (!in) give the empty key.
 template <bool NOISE>
 __device__ __forceinline__ void cand_entry(const float* cs, const uint32_t* ci, const float* grow, float coef,
-                                           uint32_t o, bool in, u64& key, float& pay) {
+                                           uint32_t o, bool in, Key& key, float& pay) {
   const float v = lds_at(cs, o);
   const int id = in ? (int)lds_at(ci, o) : 0;
   if (NOISE) {
     const float g = grow[id];  // id < n: padded keys are never buffered
-    key = in ? make_key(__builtin_fmaf(coef, g, v), id) : 0ull;
+    key = in ? make_key(__builtin_fmaf(coef, g, v), id) : kNoKey;
     pay = in ? v : 0.f;
   } else {
-    key = in ? make_key(v, id) : 0ull;
+    key = in ? make_key(v, id) : kNoKey;
     pay = 0.f;
   }
 }
@@ -181,7 +179,7 @@ __device__ __forceinline__ void flush_lane(LaneSel<KMAX, NOISE>& st, const float
 #pragma unroll 1
   for (int c0 = 0; c0 < CAP; c0 += 8) {
     if (__ballot(c0 < cnt) == 0) break;
-    u64 ch[8];
+    Key ch[8];
     float cp[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -199,8 +197,8 @@ __device__ __forceinline__ void flush_lane(LaneSel<KMAX, NOISE>& st, const float
   }
   st.off = lane0;
   if (REFRESH) {
-    const u64 kk = k == KMAX ? pair_kth_key<KMAX, NOISE>(st.top, par) : st.top.at(k - 1);
-    if (valid) st.thr = kk ? key_score(kk) : base_thr;
+    const Key kk = k == KMAX ? pair_kth_key<KMAX, NOISE>(st.top, par) : st.top.at(k - 1);
+    if (valid) st.thr = has_key(kk) ? key_score(kk) : base_thr;
   }
 }
 
@@ -219,7 +217,7 @@ __device__ __forceinline__ void flush_pair_range(LaneSel<KMAX, NOISE>& st, const
 #pragma unroll 1
   for (int c0 = 0; c0 < CAP; c0 += 8) {
     if (__ballot(c0 < cnt) == 0) break;
-    u64 ch[8];
+    Key ch[8];
     float cp[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -799,16 +797,16 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
   // arrives through v_permlane32_swap and is bitonic-merged (keys of the two
   // lanes are distinct: different key parities).
   {
-    u64 other[KMAX];
+    Key other[KMAX];
     float opay[NOISE ? KMAX : 1];
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) {
-      float lo = __uint_as_float((uint32_t)st.top.key[j]), lo2 = lo;
-      float hi = __uint_as_float((uint32_t)(st.top.key[j] >> 32)), hi2 = hi;
+      float lo = __uint_as_float(key_lo(st.top.key[j])), lo2 = lo;
+      float hi = __uint_as_float(key_hi(st.top.key[j])), hi2 = hi;
       half_swap(lo, lo2);
       half_swap(hi, hi2);
       const float plo = par ? lo : lo2, phi = par ? hi : hi2;
-      other[j] = ((u64)__float_as_uint(phi) << 32) | __float_as_uint(plo);
+      other[j] = key_of(__float_as_uint(phi), __float_as_uint(plo));
       if (NOISE) {
         float a = st.top.pay[NOISE ? j : 0], b = a;
         half_swap(a, b);
@@ -826,7 +824,7 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
     int id[KMAX];
 #pragma unroll
     for (int r = 0; r < KMAX; ++r) {
-      const u64 kk = st.top.key[r];
+      const Key kk = st.top.key[r];
       float clean, sel;
       if (NOISE) {
         clean = st.top.pay[NOISE ? r : 0];
@@ -836,10 +834,10 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
         clean *= ql;  // ql == 1 without query_scale
         sel = clean;
       }
-      if (kk == 0) clean = sel = -INFINITY;
+      if (!has_key(kk)) clean = sel = -INFINITY;
       cl[r] = clean;
       se[r] = sel;
-      id[r] = kk ? key_index(kk) : -1;
+      id[r] = has_key(kk) ? key_index(kk) : -1;
     }
     const bool vec = p.k == KMAX && ((uintptr_t)(p.out_clean + o) & 15) == 0 &&
                      ((uintptr_t)(p.out_idx + o) & 15) == 0 && (!NOISE || ((uintptr_t)(p.out_sel + o) & 15) == 0);
@@ -891,8 +889,8 @@ __global__ __launch_bounds__(64 * WPG) void score_topk_decode(ScoreParams p) {
   constexpr int TILE = VPL * kWave;
   constexpr int NG = WPG / 4;  // workgroup lists after the first reduction
   typedef typename Mfma<T>::Op Op;
-  __shared__ u64 wl[WPG][MQ][16];
-  __shared__ u64 gl[NG > 1 ? NG : 1][MQ][16];
+  __shared__ Key wl[WPG][MQ][16];
+  __shared__ Key gl[NG > 1 ? NG : 1][MQ][16];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -923,14 +921,14 @@ __global__ __launch_bounds__(64 * WPG) void score_topk_decode(ScoreParams p) {
   }
   // Query q's scores: block b0 in lanes 0-31, block b0 + 1 in lanes 32-63.
   const int idx = (b0 + (lane >> 5)) * 32 + (lane & 31);
-  u64 key[MQ];
+  Key key[MQ];
 #pragma unroll
   for (int q = 0; q < MQ; ++q) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x0[q]), __float_as_uint(x1[q]), false, false);
     const float s = __uint_as_float(r[0]);
     // padded keys and scores that are not above -inf (NaN included) are
     // never selected, as in score_topk_kernel
-    key[q] = (idx < p.n && s > -INFINITY) ? make_key(s, idx) : 0ull;
+    key[q] = (idx < p.n && s > -INFINITY) ? make_key(s, idx) : kNoKey;
   }
   w64::sort64_desc<MQ>(key, lane);
   if (lane < 16) {
@@ -940,14 +938,14 @@ __global__ __launch_bounds__(64 * WPG) void score_topk_decode(ScoreParams p) {
   __syncthreads();
   // lane i of a reducing wave loads entry i % 16 of list i / 16 of its group
   // of four, lists 1 and 3 reversed; lists past the end are empty
-  auto load4 = [&](const u64 (*lists)[MQ][16], int first, int count) __attribute__((always_inline)) {
+  auto load4 = [&](const Key (*lists)[MQ][16], int first, int count) __attribute__((always_inline)) {
     const int t = lane >> 4, e = lane & 15;
     const int ent = (t & 1) ? 15 - e : e;
 const int li = min(first + t, count - 1);
 #pragma unroll
     for (int q = 0; q < MQ; ++q) {
-      const u64 kk = lists[li][q][ent];
-      key[q] = first + t < count ? kk : 0ull;
+      const Key kk = lists[li][q][ent];
+      key[q] = first + t < count ? kk : kNoKey;
     }
     w64::best16_of4<MQ>(key, lane);
   };
@@ -976,12 +974,12 @@ const int li = min(first + t, count - 1);
     for (int q = 0; q < MQ; ++q) {
       if (q < p.M) {
         const float qlq = qls[q];
-        const u64 kk = key[q];
+        const Key kk = key[q];
         float clean = key_score(kk) * Tv;
         clean *= qlq;  // 1 without query_scale
         const int64_t o = (((int64_t)split * p.M + q) * p.HC + hc) * p.k + lane;
-        p.out_clean[o] = kk ? clean : -INFINITY;
-        p.out_idx[o] = kk ? key_index(kk) : -1;
+        p.out_clean[o] = has_key(kk) ? clean : -INFINITY;
+        p.out_idx[o] = has_key(kk) ? key_index(kk) : -1;
       }
     }
   }
@@ -1033,12 +1031,12 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
   const int HC = 2 * p.H;
   const float* lsel = p.sel != nullptr ? p.sel : p.clean;
 
-  u64 lk[2];
+  Key lk[2];
   float lc[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const int hc = 2 * h + c;
-    u64 acc = 0;
+    Key acc = kNoKey;
     float pay = 0.f;
     for (int s = 0; s < p.S; ++s) {
       const bool ok = live && r < k;
@@ -1046,7 +1044,7 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
       const int id0 = p.idx[o];
       const float sl0 = lsel[o], cc0 = p.clean[o];
       const int id = ok ? id0 : -1;
-      const u64 kk = id >= 0 ? make_key(sl0, id) : 0ull;
+      const Key kk = id >= 0 ? make_key(sl0, id) : kNoKey;
       const float cc = ok ? cc0 : 0.f;
       if (s == 0) {
         acc = kk;
@@ -1059,11 +1057,11 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
     lc[c] = pay;
     if (p.S > 1 && live && r < k) {
       const int64_t so = (m * HC + hc) * k + r;
-      p.sub_idx[so] = acc ? key_index(acc) : -1;
-      p.sub_scores[so] = acc ? pay : -INFINITY;
+      p.sub_idx[so] = has_key(acc) ? key_index(acc) : -1;
+      p.sub_scores[so] = has_key(acc) ? pay : -INFINITY;
     }
   }
-  const bool a_ok = lk[0] != 0ull, b_ok = lk[1] != 0ull;
+  const bool a_ok = has_key(lk[0]), b_ok = has_key(lk[1]);
   const float a_sel = a_ok ? key_score(lk[0]) : -INFINITY;
   const float b_sel = b_ok ? key_score(lk[1]) : -INFINITY;
   const int a_id = a_ok ? key_index(lk[0]) : 0;
@@ -1074,14 +1072,14 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
   const float a0 = __shfl(a_sel, base);
   const float a0c = __shfl(a_cl, base);
   const bool a0_ok = __shfl((int)a_ok, base) != 0;
-  u64 acc = (r < k && a0_ok && b_ok) ? make_key(a0 + b_sel, r) : 0ull;
+  Key acc = (r < k && a0_ok && b_ok) ? make_key(a0 + b_sel, r) : kNoKey;
   float pay = a0c + b_cl;
   // rows 1 .. k/2-1: (i, j) for j < k/(i+1)
   for (int i = 1; i < k / 2; ++i) {
     const float ai = __shfl(a_sel, base + i);
     const float aic = __shfl(a_cl, base + i);
     const bool ai_ok = __shfl((int)a_ok, base + i) != 0;
-    const u64 cand = (r < k / (i + 1) && ai_ok && b_ok) ? make_key(ai + b_sel, i * k + r) : 0ull;
+    const Key cand = (r < k / (i + 1) && ai_ok && b_ok) ? make_key(ai + b_sel, i * k + r) : kNoKey;
     group_merge<G>(acc, pay, cand, aic + b_cl, r, base);
   }
   // rows max(1, k/2) .. k-1: only (i, 0) can reach the top k
@@ -1094,12 +1092,12 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
     const float ar = __shfl(a_sel, src);
     const float arc = __shfl(a_cl, src);
     const bool ar_ok = __shfl((int)a_ok, src) != 0;
-    const u64 cand = (r < k - i0 && ar_ok && b0_ok) ? make_key(ar + b0, (i0 + r) * k) : 0ull;
+    const Key cand = (r < k - i0 && ar_ok && b0_ok) ? make_key(ar + b0, (i0 + r) * k) : kNoKey;
     group_merge<G>(acc, pay, cand, arc + b0c, r, base);
   }
 
   // lane r < k holds the rank-r slot
-  const int flat = acc ? key_index(acc) : 0;
+  const int flat = has_key(acc) ? key_index(acc) : 0;
   const int ra = min(flat / k, G - 1), rb = flat % k;
   int ia = __shfl(a_id, base + ra);
   int ib = __shfl(b_id, base + rb);
@@ -1128,11 +1126,11 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
 // live row.
 // The lane's slot id (in [0, n*n)) and weight are also returned in slot_out
 // and w_out, for a value read fused behind the pair stage.
-__device__ __forceinline__ void pair_tail_k16(const PairParams& p, const u64 (&lk)[2], const float (&lc)[2],
+__device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&lk)[2], const float (&lc)[2],
                                               bool live, int64_t mh, int lane, int r, int& slot_out,
                                               float& w_out) {
   constexpr int K = 16;
-  const bool a_ok = lk[0] != 0ull, b_ok = lk[1] != 0ull;
+  const bool a_ok = has_key(lk[0]), b_ok = has_key(lk[1]);
   const float a_sel = a_ok ? key_score(lk[0]) : -INFINITY;
   const float b_sel = b_ok ? key_score(lk[1]) : -INFINITY;
   const int a_id = a_ok ? key_index(lk[0]) : 0;
@@ -1145,12 +1143,12 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const u64 (&l
   // (i, 0) of rows 8..15 at lane i - 8.  They are merged as a tree, so the
   // merges of one level are independent and fill each other's exchange
   // latencies.
-  u64 L[9];
+  Key L[9];
   float P[9];
 #define MPL_PAIR_ROW(I)                                                                                 \
   {                                                                                                     \
     const float ai = g16::bcastf<I>(a_sel), aic = g16::bcastf<I>(a_cl), aik = g16::bcastf<I>(aok);    \
-    L[I] = (r < K / (I + 1) && aik != 0.f && b_ok) ? make_key(ai + b_sel, I * K + r) : 0ull;           \
+    L[I] = (r < K / (I + 1) && aik != 0.f && b_ok) ? make_key(ai + b_sel, I * K + r) : kNoKey;           \
     P[I] = aic + b_cl;                                                                                  \
   }
   MPL_PAIR_ROW(0) MPL_PAIR_ROW(1) MPL_PAIR_ROW(2) MPL_PAIR_ROW(3) MPL_PAIR_ROW(4) MPL_PAIR_ROW(5)
@@ -1162,7 +1160,7 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const u64 (&l
     const float ar = __uint_as_float(g16::shl8(__float_as_uint(a_sel)));
     const float arc = __uint_as_float(g16::shl8(__float_as_uint(a_cl)));
     const float ark = __uint_as_float(g16::shl8(__float_as_uint(aok)));
-    L[8] = (r < 8 && ark != 0.f && b0_ok) ? make_key(ar + b0, (8 + r) * K) : 0ull;
+    L[8] = (r < 8 && ark != 0.f && b0_ok) ? make_key(ar + b0, (8 + r) * K) : kNoKey;
     P[8] = arc + b0c;
   }
 #pragma unroll
@@ -1171,19 +1169,19 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const u64 (&l
   g16::merge(L[4], P[4], L[6], P[6], r);
   g16::merge(L[0], P[0], L[4], P[4], r);
   g16::merge(L[0], P[0], L[8], P[8], r);
-  const u64 acc = L[0];
+  const Key acc = L[0];
   const float pay = P[0];
 
   // lane r holds the rank-r slot
-  const int flat = acc ? key_index(acc) : 0;
+  const int flat = has_key(acc) ? key_index(acc) : 0;
   const int base = lane - r;
   int ia = __shfl(a_id, base + flat / K);
   int ib = __shfl(b_id, base + flat % K);
   ia = (ia >= 0 && ia < p.n) ? ia : 0;  // ids come from keys < n; guards non-finite inputs
   ib = (ib >= 0 && ib < p.n) ? ib : 0;
-  const float sc = acc ? pay : -INFINITY;
+  const float sc = has_key(acc) ? pay : -INFINITY;
   const float mx = g16::rmax(sc);
-  const float e = acc ? expf(sc - mx) : 0.f;
+  const float e = has_key(acc) ? expf(sc - mx) : 0.f;
   const float sum = g16::rsum(e);
   slot_out = ia * p.n + ib;
   w_out = e / sum;
@@ -1197,7 +1195,7 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const u64 (&l
 
 // The two codebooks' final lists of row mh (lane r gets rank r of lk[c] and
 // its clean score lc[c]): one split list loaded, or S lists merged.
-__device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, int64_t mh, int r, u64 (&lk)[2],
+__device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, int64_t mh, int r, Key (&lk)[2],
                                                float (&lc)[2]) {
   constexpr int K = 16;
   const int64_t m = live ? mh / p.H : 0;
@@ -1219,7 +1217,7 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
       float sl[1] = {lsel[o0[c]]}, cc[1] = {p.clean[o0[c]]};
       pin_loaded(id, sl, cc);
       lc[c] = cc[0];
-      lk[c] = (live && id[0] >= 0) ? make_key(sl[0], id[0]) : 0ull;
+      lk[c] = (live && id[0] >= 0) ? make_key(sl[0], id[0]) : kNoKey;
     }
   } else {
     constexpr int B = 8;
@@ -1243,7 +1241,7 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
 #pragma unroll
         for (int t = 0; t < B; ++t) {
           if (s0 + t < p.S) {  // uniform
-            const u64 kk = (live && id[c][t] >= 0) ? make_key(sl[c][t], id[c][t]) : 0ull;
+            const Key kk = (live && id[c][t] >= 0) ? make_key(sl[c][t], id[c][t]) : kNoKey;
             if (s0 + t == 0) {
               lk[c] = kk;
               lc[c] = cc[c][t];
@@ -1256,8 +1254,8 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
 #pragma unroll
     for (int c = 0; c < 2; ++c)
       if (live) {
-        p.sub_idx[o0[c]] = lk[c] ? key_index(lk[c]) : -1;
-        p.sub_scores[o0[c]] = lk[c] ? lc[c] : -INFINITY;
+        p.sub_idx[o0[c]] = has_key(lk[c]) ? key_index(lk[c]) : -1;
+        p.sub_scores[o0[c]] = has_key(lk[c]) ? lc[c] : -INFINITY;
       }
   }
 }
@@ -1267,7 +1265,7 @@ __global__ __launch_bounds__(256) void pair_kernel_k16(PairParams p) {
   const int r = lane & 15;
   const int64_t mh = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
   const bool live = mh < p.M * p.H;  // dead rows still join the exchanges
-  u64 lk[2];
+  Key lk[2];
   float lc[2];
   pair_lists_k16(p, live, mh, r, lk, lc);
   int slot;
@@ -1294,7 +1292,7 @@ __global__ __launch_bounds__(256) void pair_read_k16(PairParams p, ReadParams rp
   const int r = lane & 15;
   const int64_t mh = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
   const bool live = mh < p.M * 4;  // H = 4: a wave is live or dead as a whole
-  u64 lk[2];
+  Key lk[2];
   float lc[2];
   pair_lists_k16(p, live, mh, r, lk, lc);
   int slot;
@@ -1348,12 +1346,12 @@ __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
     cc[t] = p.clean[o];
   }
   pin_loaded(id, sl, cc);
-  u64 acc = 0;
+  Key acc = kNoKey;
   float pay = 0.f;
 #pragma unroll
   for (int t = 0; t < kMergeChunk; ++t) {
     const bool in = s2 * kMergeChunk + t < p.S;  // uniform per row
-    const u64 kk = (in && id[t] >= 0) ? make_key(sl[t], id[t]) : 0ull;
+    const Key kk = (in && id[t] >= 0) ? make_key(sl[t], id[t]) : kNoKey;
     if (t == 0) {
       acc = kk;
       pay = cc[t];
@@ -1363,9 +1361,9 @@ __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
   }
   if (live) {
     const int64_t o = ((int64_t)s2 * p.rows + row) * K + r;
-    p.out_idx[o] = acc ? key_index(acc) : -1;
-    p.out_clean[o] = acc ? pay : -INFINITY;
-    if (p.out_sel != nullptr) p.out_sel[o] = acc ? key_score(acc) : -INFINITY;
+    p.out_idx[o] = has_key(acc) ? key_index(acc) : -1;
+    p.out_clean[o] = has_key(acc) ? pay : -INFINITY;
+    if (p.out_sel != nullptr) p.out_sel[o] = has_key(acc) ? key_score(acc) : -INFINITY;
   }
 }
 
@@ -1380,7 +1378,7 @@ constexpr int kWideMaxSplits = kMergeChunk * kMergeChunk;
 
 __global__ __launch_bounds__(256) void pair_wide_k16(PairParams p) {
   constexpr int K = 16;
-  __shared__ u64 skey[16][K];
+  __shared__ Key skey[16][K];
   __shared__ float spay[16][K];
   const int lane = threadIdx.x & 63;
   const int r = lane & 15;
@@ -1403,12 +1401,12 @@ __global__ __launch_bounds__(256) void pair_wide_k16(PairParams p) {
     cc[t] = p.clean[o];
   }
   pin_loaded(id, sl, cc);
-  u64 acc = 0;
+  Key acc = kNoKey;
   float pay = 0.f;
 #pragma unroll
   for (int t = 0; t < kMergeChunk; ++t) {
     const bool in = chunk * kMergeChunk + t < p.S;  // uniform per row
-    const u64 kk = (in && id[t] >= 0) ? make_key(sl[t], id[t]) : 0ull;
+    const Key kk = (in && id[t] >= 0) ? make_key(sl[t], id[t]) : kNoKey;
     if (t == 0) {
       acc = kk;
       pay = cc[t];
@@ -1422,14 +1420,14 @@ __global__ __launch_bounds__(256) void pair_wide_k16(PairParams p) {
   if (chunk == 0) {  // rows 0 and 8 read rows 1..7 and 9..15 and rewrite only their own entries
 #pragma unroll
     for (int t = 1; t < kMergeChunk; ++t) g16::merge(acc, pay, skey[g + t][r], spay[g + t][r], r);
-    p.sub_idx[o0] = acc ? key_index(acc) : -1;
-    p.sub_scores[o0] = acc ? pay : -INFINITY;
+    p.sub_idx[o0] = has_key(acc) ? key_index(acc) : -1;
+    p.sub_scores[o0] = has_key(acc) ? pay : -INFINITY;
     skey[g][r] = acc;
     spay[g][r] = pay;
   }
   __syncthreads();
   if (g == 0) {
-    const u64 lk[2] = {skey[0][r], skey[8][r]};
+    const Key lk[2] = {skey[0][r], skey[8][r]};
     const float lc[2] = {spay[0][r], spay[8][r]};
     int slot;
     float w;
@@ -1448,7 +1446,7 @@ __global__ __launch_bounds__(256) void pair_wide_k16(PairParams p) {
 template <typename V, int VR, bool NT>
 __global__ __launch_bounds__(1024) void pair_wide_read_k16(PairParams p, ReadParams rp) {
   constexpr int K = 16;
-  __shared__ u64 skey[4][16][K];
+  __shared__ Key skey[4][16][K];
   __shared__ float spay[4][16][K];
   __shared__ int srow_slot[4 * K];
   __shared__ float srow_w[4 * K];
@@ -1474,12 +1472,12 @@ __global__ __launch_bounds__(1024) void pair_wide_read_k16(PairParams p, ReadPar
     cc[i] = p.clean[o];
   }
   pin_loaded(id, sl, cc);
-  u64 acc = 0;
+  Key acc = kNoKey;
   float pay = 0.f;
 #pragma unroll
   for (int i = 0; i < kMergeChunk; ++i) {
     const bool in = chunk * kMergeChunk + i < p.S;  // uniform per row
-    const u64 kk = (in && id[i] >= 0) ? make_key(sl[i], id[i]) : 0ull;
+    const Key kk = (in && id[i] >= 0) ? make_key(sl[i], id[i]) : kNoKey;
     if (i == 0) {
       acc = kk;
       pay = cc[i];
@@ -1493,14 +1491,14 @@ __global__ __launch_bounds__(1024) void pair_wide_read_k16(PairParams p, ReadPar
   if (chunk == 0) {  // rows 0 and 8 of each quarter read rows 1..7 and 9..15 and rewrite only their own
 #pragma unroll
     for (int i = 1; i < kMergeChunk; ++i) g16::merge(acc, pay, skey[h][g + i][r], spay[h][g + i][r], r);
-    p.sub_idx[o0] = acc ? key_index(acc) : -1;
-    p.sub_scores[o0] = acc ? pay : -INFINITY;
+    p.sub_idx[o0] = has_key(acc) ? key_index(acc) : -1;
+    p.sub_scores[o0] = has_key(acc) ? pay : -INFINITY;
     skey[h][g][r] = acc;
     spay[h][g][r] = pay;
   }
   __syncthreads();
   if (g == 0) {  // lanes 0-15 of the quarter's first wave
-    const u64 lk[2] = {skey[h][0][r], skey[h][8][r]};
+    const Key lk[2] = {skey[h][0][r], skey[h][8][r]};
     const float lc[2] = {spay[h][0][r], spay[h][8][r]};
     int slot;
     float w;
@@ -1552,9 +1550,9 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
   constexpr int HG = GROUPS / 4;     // row groups of one head
   constexpr int G1 = SC / 8;         // groups of four lists per wave in step 1
   constexpr int GPC = G1 / 2;        // groups per codebook in step 2
-  __shared__ u64 l1[4][2][2 * G1][K];  // [head][codebook][list][rank] after step 1
-  __shared__ u64 l2[4][G1][K];         // [head][list] within step 2
-  __shared__ u64 pab[4][2][K];         // [head][codebook] final lists
+  __shared__ Key l1[4][2][2 * G1][K];  // [head][codebook][list][rank] after step 1
+  __shared__ Key l2[4][G1][K];         // [head][list] within step 2
+  __shared__ Key pab[4][2][K];         // [head][codebook] final lists
   __shared__ float srow_w[4 * K];
   __shared__ uint4 rows[GROUPS][kWave];
 
@@ -1579,11 +1577,11 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
       id[grp] = p.idx[o];
       cl[grp] = p.clean[o];
     }
-    u64 key[G1];
+    Key key[G1];
 #pragma unroll
     for (int grp = 0; grp < G1; ++grp) {
       const int s = (SC / 2) * (sub & 1) + 4 * grp + t;
-      key[grp] = (s < p.S && id[grp] >= 0) ? make_key(cl[grp], id[grp]) : 0ull;
+      key[grp] = (s < p.S && id[grp] >= 0) ? make_key(cl[grp], id[grp]) : kNoKey;
     }
     w64::best16_of4<G1>(key, lane);
     if (lane < K) {
@@ -1595,7 +1593,7 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
   if (wave < 4) {
     const int h = wave;
     // step 2a: group g holds lists 4 * (g % GPC) + t of codebook g / GPC
-    u64 key[G1];
+    Key key[G1];
 #pragma unroll
     for (int g = 0; g < G1; ++g) key[g] = l1[h][g / GPC][4 * (g % GPC) + t][ent];
     w64::best16_of4<G1>(key, lane);
@@ -1605,26 +1603,26 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
     }
     // step 2b: each codebook's GPC lists to one, codebook 0 in lanes 0-15
     // and codebook 1 in lanes 32-47
-    u64 fk;
+    Key fk;
     if constexpr (GPC == 2) {
       // lanes 0-31 hold codebook 0's two lists, lanes 32-63 codebook 1's
       // (second of each reversed): one bitonic split and a 16-lane merger
-      u64 v[1] = {l2[h][t][ent]};
-      const u64 o = w64::xr64<16>(v[0], lane);
+      Key v[1] = {l2[h][t][ent]};
+      const Key o = w64::xr64<16>(v[0], lane);
       v[0] = o > v[0] ? o : v[0];
       w64::merge_down<8, 1>(v, lane, true);
       fk = v[0];
     } else {
-      u64 v[2] = {l2[h][t][ent], l2[h][4 + t][ent]};  // a group of four per codebook
+      Key v[2] = {l2[h][t][ent], l2[h][4 + t][ent]};  // a group of four per codebook
       w64::best16_of4<2>(v, lane);
-      const u64 b = w64::xr64<32>(v[1], lane);  // codebook 1's list to lanes 32-47
+      const Key b = w64::xr64<32>(v[1], lane);  // codebook 1's list to lanes 32-47
       fk = (lane & 32) ? b : v[0];
     }
     if ((lane & 16) == 0) {  // lanes 0-15: codebook 2h, lanes 32-47: 2h + 1
       const int cb = lane >> 5;
       const int64_t o0 = (m * HC + 2 * h + cb) * K + e;
-      p.sub_idx[o0] = fk ? key_index(fk) : -1;
-      p.sub_scores[o0] = fk ? key_score(fk) : -INFINITY;
+      p.sub_idx[o0] = has_key(fk) ? key_index(fk) : -1;
+      p.sub_scores[o0] = has_key(fk) ? key_score(fk) : -INFINITY;
       pab[h][cb][e] = fk;
     }
     // the pair stage: lane l < 50 takes candidate (i, j), the l-th pair with
@@ -1639,22 +1637,22 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
       pj = (!found && !here) ? pj - cnt : pj;
       found = found || here;
     }
-    const u64 ka = pab[h][0][pi], kb = pab[h][1][found ? pj : 0];
-    const bool ok = found && ka != 0ull && kb != 0ull;
-    u64 pk[1] = {ok ? make_key(key_score(ka) + key_score(kb), pi * K + pj) : 0ull};
+    const Key ka = pab[h][0][pi], kb = pab[h][1][found ? pj : 0];
+    const bool ok = found && has_key(ka) && has_key(kb);
+    Key pk[1] = {ok ? make_key(key_score(ka) + key_score(kb), pi * K + pj) : kNoKey};
     w64::sort64_desc<1>(pk, lane);
-    const u64 acc = pk[0];
+    const Key acc = pk[0];
     // lane r < 16 holds the rank-r pair (as pair_tail_k16)
-    const int flat = acc ? key_index(acc) : 0;
-    const u64 wa = pab[h][0][flat / K], wb = pab[h][1][flat % K];
-    int ia = wa ? key_index(wa) : 0;
-    int ib = wb ? key_index(wb) : 0;
+    const int flat = has_key(acc) ? key_index(acc) : 0;
+    const Key wa = pab[h][0][flat / K], wb = pab[h][1][flat % K];
+    int ia = has_key(wa) ? key_index(wa) : 0;
+    int ib = has_key(wb) ? key_index(wb) : 0;
     ia = (ia >= 0 && ia < p.n) ? ia : 0;  // ids come from keys < n; guards non-finite inputs
     ib = (ib >= 0 && ib < p.n) ? ib : 0;
-    const float pay = (wa ? key_score(wa) : -INFINITY) + (wb ? key_score(wb) : -INFINITY);
-    const float sc = acc ? pay : -INFINITY;
+    const float pay = (has_key(wa) ? key_score(wa) : -INFINITY) + (has_key(wb) ? key_score(wb) : -INFINITY);
+    const float sc = has_key(acc) ? pay : -INFINITY;
     const float mx = g16::rmax(sc);
-    const float ex = acc ? expf(sc - mx) : 0.f;
+    const float ex = has_key(acc) ? expf(sc - mx) : 0.f;
     const float sum = g16::rsum(ex);
     const int slot = ia * p.n + ib;
     const float w = ex / sum;

@@ -1,10 +1,19 @@
 // Exact top-k building blocks on 64-bit keys.
 //
-// A candidate (score, index) is packed as
-//     key = (orderable(score) << 32) | (0xFFFFFFFF - index)
-// so that unsigned key order is (score descending, index ascending): the
-// order of lax.top_k, ties going to the lowest index.  Key 0 is below every
-// real candidate and marks an empty slot.
+// A candidate (score, index) is packed into the bits of a double, the fp32
+// score's bits in the high word and the complemented index below them, so
+// that the order of doubles is (score descending, index ascending): the order
+// of lax.top_k, ties going to the lowest index.  A double orders by sign and
+// magnitude as a float does, whatever its bits mean, so the score's bits keep
+// their order there; below a negative score the index is stored as it is (a
+// larger magnitude is a smaller key).  No score but a NaN with a payload of
+// all ones makes a double that is not finite, and kNoKey (score -inf, below
+// every index) marks an empty slot and loses to every real candidate.
+//
+// Why doubles: gfx950 compare-exchanges two of them in registers with one
+// v_max_f64 and one v_min_f64 (15.5 cycles a wave on a SIMD), exactly
+// (denormal keys included).  The same exchange on 64-bit integers is a
+// v_cmp_lt_u64 and four v_cndmask with wait states between them (98 cycles).
 //
 // TopList<KMAX> keeps the best KMAX keys sorted descending in registers.
 // Candidates are merged in chunks of 8: an optimal 19-comparator network
@@ -29,30 +38,42 @@ __device__ __forceinline__ float from_orderable(uint32_t u) {
   return __uint_as_float(b);
 }
 
-__device__ __forceinline__ u64 make_key(float s, int idx) {
-  return ((u64)orderable(s) << 32) | (u64)(0xFFFFFFFFu - (uint32_t)idx);
+typedef double Key;
+constexpr Key kNoKey = __builtin_bit_cast(Key, 0xFF800000FFFFFFFFull);
+
+__device__ __forceinline__ u64 key_bits(Key k) { return __builtin_bit_cast(u64, k); }
+__device__ __forceinline__ Key key_of(uint32_t hi, uint32_t lo) {
+  return __builtin_bit_cast(Key, ((u64)hi << 32) | (u64)lo);
+}
+__device__ __forceinline__ uint32_t key_hi(Key k) { return (uint32_t)(key_bits(k) >> 32); }
+__device__ __forceinline__ uint32_t key_lo(Key k) { return (uint32_t)key_bits(k); }
+
+__device__ __forceinline__ Key make_key(float s, int idx) {
+  const uint32_t b = __float_as_uint(s + 0.0f);  // -0 -> +0
+  return key_of(b, ~(uint32_t)idx ^ (uint32_t)((int)b >> 31));
 }
 
-__device__ __forceinline__ float key_score(u64 k) { return from_orderable((uint32_t)(k >> 32)); }
-__device__ __forceinline__ int key_index(u64 k) { return (int)(0xFFFFFFFFu - (uint32_t)k); }
+__device__ __forceinline__ bool has_key(Key k) { return k > kNoKey; }
+__device__ __forceinline__ float key_score(Key k) { return __uint_as_float(key_hi(k)); }
+__device__ __forceinline__ int key_index(Key k) { return (int)~(key_lo(k) ^ (uint32_t)((int)key_hi(k) >> 31)); }
 
 // Compare-exchange, larger key to `a`.
 template <bool PAY>
-__device__ __forceinline__ void cex(u64& a, u64& b, float& pa, float& pb) {
-  const bool sw = a < b;
-  const u64 t = sw ? b : a;
-  b = sw ? a : b;
-  a = t;
+__device__ __forceinline__ void cex(Key& a, Key& b, float& pa, float& pb) {
   if (PAY) {
+    const bool sw = a < b;
     const float q = sw ? pb : pa;
     pb = sw ? pa : pb;
     pa = q;
   }
+  const Key t = __builtin_fmax(a, b);
+  b = __builtin_fmin(a, b);
+  a = t;
 }
 
 // Sorts 8 keys descending (optimal 19-comparator network).
 template <bool PAY>
-__device__ __forceinline__ void sort8(u64* c, float* p) {
+__device__ __forceinline__ void sort8(Key* c, float* p) {
 #define MPL_CE(i, j) cex<PAY>(c[i], c[j], p[PAY ? i : 0], p[PAY ? j : 0])
   MPL_CE(0, 2); MPL_CE(1, 3); MPL_CE(4, 6); MPL_CE(5, 7);
   MPL_CE(0, 4); MPL_CE(1, 5); MPL_CE(2, 6); MPL_CE(3, 7);
@@ -65,25 +86,24 @@ __device__ __forceinline__ void sort8(u64* c, float* p) {
 
 template <int KMAX, bool PAY>
 struct TopList {
-  u64 key[KMAX];
+  Key key[KMAX];
   float pay[PAY ? KMAX : 1];
 
   __device__ __forceinline__ void init() {
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) key[j] = 0;
+    for (int j = 0; j < KMAX; ++j) key[j] = kNoKey;
 #pragma unroll
     for (int j = 0; j < (PAY ? KMAX : 1); ++j) pay[j] = 0.f;
   }
 
   // Merge a sorted (descending) run of CN <= KMAX keys.
   template <int CN>
-  __device__ __forceinline__ void merge(const u64* c, const float* cp) {
+  __device__ __forceinline__ void merge(const Key* c, const float* cp) {
 #pragma unroll
     for (int i = KMAX - CN; i < KMAX; ++i) {
-      const u64 b = c[KMAX - 1 - i];
-      const bool take = b > key[i];
-      key[i] = take ? b : key[i];
-      if (PAY) pay[PAY ? i : 0] = take ? cp[PAY ? KMAX - 1 - i : 0] : pay[PAY ? i : 0];
+      const Key b = c[KMAX - 1 - i];
+      if (PAY) pay[PAY ? i : 0] = b > key[i] ? cp[PAY ? KMAX - 1 - i : 0] : pay[PAY ? i : 0];
+      key[i] = __builtin_fmax(b, key[i]);
     }
     // Affine stage counter: every index below is a compile-time constant,
     // so the list stays in registers.
@@ -101,11 +121,11 @@ struct TopList {
   // Key at runtime position r (< KMAX).  Written as and/or of masked
   // entries: a select chain on r would be folded into a dynamically indexed
   // load, which forces the whole list out of registers into scratch.
-  __device__ __forceinline__ u64 at(int r) const {
+  __device__ __forceinline__ Key at(int r) const {
     u64 t = 0;
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) t |= key[j] & (0ull - (u64)(j == r));
-    return t;
+    for (int j = 0; j < KMAX; ++j) t |= key_bits(key[j]) & (0ull - (u64)(j == r));
+    return __builtin_bit_cast(Key, t);
   }
 };
 
@@ -117,25 +137,25 @@ namespace mpl {
 // A group of G lanes (16 or 32, aligned within the wave) holds one sorted
 // list: the lane of rank r (= lane % G) holds the r-th best key.
 
-__device__ __forceinline__ u64 shfl_u64(u64 v, int src) {
-  const uint32_t lo = __shfl((uint32_t)v, src);
-  const uint32_t hi = __shfl((uint32_t)(v >> 32), src);
-  return ((u64)hi << 32) | lo;
+__device__ __forceinline__ Key shfl_key(Key v, int src) {
+  const uint32_t lo = __shfl(key_lo(v), src);
+  const uint32_t hi = __shfl(key_hi(v), src);
+  return key_of(hi, lo);
 }
 
 template <int G>
-__device__ __forceinline__ u64 shfl_xor_u64(u64 v, int mask) {
-  const uint32_t lo = __shfl_xor((uint32_t)v, mask, G);
-  const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), mask, G);
-  return ((u64)hi << 32) | lo;
+__device__ __forceinline__ Key shfl_xor_key(Key v, int mask) {
+  const uint32_t lo = __shfl_xor(key_lo(v), mask, G);
+  const uint32_t hi = __shfl_xor(key_hi(v), mask, G);
+  return key_of(hi, lo);
 }
 
 // acc <- best G of (acc, b), both sorted descending across the group; the
 // float payload follows its key.  Bitonic split + G-wide bitonic merger.
 template <int G>
-__device__ __forceinline__ void group_merge(u64& acc, float& pay, u64 b, float bp, int r, int base) {
+__device__ __forceinline__ void group_merge(Key& acc, float& pay, Key b, float bp, int r, int base) {
   const int src = base + (G - 1 - r);
-  const u64 br = shfl_u64(b, src);
+  const Key br = shfl_key(b, src);
   const float bpr = __shfl(bp, src);
   const bool take = br > acc;
   acc = take ? br : acc;
@@ -144,7 +164,7 @@ __device__ __forceinline__ void group_merge(u64& acc, float& pay, u64 b, float b
 #pragma unroll
   for (int st = 0; st < kStages; ++st) {
     const int s = (G / 2) >> st;
-    const u64 o = shfl_xor_u64<G>(acc, s);
+    const Key o = shfl_xor_key<G>(acc, s);
     const float op = __shfl_xor(pay, s, G);
     const bool other = (o > acc) != ((r & s) != 0);  // as in g16::merge
     acc = other ? o : acc;
@@ -199,8 +219,8 @@ __device__ __forceinline__ uint32_t shl8(uint32_t v) {
 }
 
 template <int S>
-__device__ __forceinline__ u64 xr64(u64 v) {
-  return ((u64)xr<S>((uint32_t)(v >> 32)) << 32) | xr<S>((uint32_t)v);
+__device__ __forceinline__ Key xr64(Key v) {
+  return key_of(xr<S>(key_hi(v)), xr<S>(key_lo(v)));
 }
 template <int S>
 __device__ __forceinline__ float xrf(float v) {
@@ -216,17 +236,17 @@ __device__ __forceinline__ float bcastf(float v) {
 // mirrored b, then a 4-stage bitonic merger.  In a stage the lower lane of a
 // pair keeps the larger key and the upper lane the smaller: the upper lane
 // takes its partner's key unless that key is larger, so one compare serves
-// both (equal keys are only the empty key 0, whose swap changes nothing that
+// both (equal keys are only the empty key, whose swap changes nothing that
 // is output).
-__device__ __forceinline__ void merge(u64& acc, float& pay, u64 b, float bp, int r) {
-  const u64 br = ((u64)mirror((uint32_t)(b >> 32)) << 32) | mirror((uint32_t)b);
+__device__ __forceinline__ void merge(Key& acc, float& pay, Key b, float bp, int r) {
+  const Key br = key_of(mirror(key_hi(b)), mirror(key_lo(b)));
   const float bpr = __uint_as_float(mirror(__float_as_uint(bp)));
   const bool take = br > acc;
   acc = take ? br : acc;
   pay = take ? bpr : pay;
 #define MPL_G16_STAGE(S)                                  \
   {                                                       \
-    const u64 o = xr64<S>(acc);                           \
+    const Key o = xr64<S>(acc);                           \
     const float op = xrf<S>(pay);                         \
     const bool upper = (r & S) != 0;                      \
     const bool other = (o > acc) != upper;                \
@@ -262,7 +282,7 @@ namespace mpl {
 // Exchanges with lane ^ S across the 64-lane wave, on the VALU only: DPP
 // inside 16-lane rows for S < 16 (xor 4 as a shift left and a shift right
 // on alternate banks of 4 lanes), v_permlane16_swap / v_permlane32_swap for
-// 16 and 32.  Bitonic sorts and merges of u64 keys (the order of make_key).
+// 16 and 32.  Bitonic sorts and merges of keys (the order of make_key).
 namespace w64 {
 
 template <int S>
@@ -290,17 +310,17 @@ __device__ __forceinline__ uint32_t xr(uint32_t v, int lane) {
 }
 
 template <int S>
-__device__ __forceinline__ u64 xr64(u64 v, int lane) {
-  return ((u64)xr<S>((uint32_t)(v >> 32), lane) << 32) | xr<S>((uint32_t)v, lane);
+__device__ __forceinline__ Key xr64(Key v, int lane) {
+  return key_of(xr<S>(key_hi(v), lane), xr<S>(key_lo(v), lane));
 }
 
 // One compare-exchange stage with lane ^ S on N independent lists: the lane
 // keeps the larger key when keep_max, else the smaller.
 template <int S, int N>
-__device__ __forceinline__ void stage(u64 (&v)[N], int lane, bool keep_max) {
+__device__ __forceinline__ void stage(Key (&v)[N], int lane, bool keep_max) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const u64 o = xr64<S>(v[i], lane);
+    const Key o = xr64<S>(v[i], lane);
     v[i] = ((o > v[i]) == keep_max) ? o : v[i];
   }
 }
@@ -308,14 +328,14 @@ __device__ __forceinline__ void stage(u64 (&v)[N], int lane, bool keep_max) {
 // Bitonic merge of stages S, S/2, ..., 1: each aligned group of 2S lanes
 // holding a bitonic sequence ends sorted, descending where desc.
 template <int S, int N>
-__device__ __forceinline__ void merge_down(u64 (&v)[N], int lane, bool desc) {
+__device__ __forceinline__ void merge_down(Key (&v)[N], int lane, bool desc) {
   stage<S, N>(v, lane, ((lane & S) == 0) == desc);
   if constexpr (S > 1) merge_down<S / 2, N>(v, lane, desc);
 }
 
 // Sorts the wave's 64 keys of each list descending: lane r ends with rank r.
 template <int N>
-__device__ __forceinline__ void sort64_desc(u64 (&v)[N], int lane) {
+__device__ __forceinline__ void sort64_desc(Key (&v)[N], int lane) {
   merge_down<1, N>(v, lane, (lane & 2) == 0);
   merge_down<2, N>(v, lane, (lane & 4) == 0);
   merge_down<4, N>(v, lane, (lane & 8) == 0);
@@ -328,16 +348,16 @@ __device__ __forceinline__ void sort64_desc(u64 (&v)[N], int lane) {
 // i / 16, lists 1 and 3 in reverse order (so lanes 0-31 and 32-63 are each
 // a bitonic sequence).  Lanes 0-15 end with the best 16, descending.
 template <int N>
-__device__ __forceinline__ void best16_of4(u64 (&v)[N], int lane) {
+__device__ __forceinline__ void best16_of4(Key (&v)[N], int lane) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {  // lists 0+1 -> lanes 0-15, lists 2+3 -> lanes 32-47 (bitonic split)
-    const u64 o = xr64<16>(v[i], lane);
+    const Key o = xr64<16>(v[i], lane);
     v[i] = o > v[i] ? o : v[i];
   }
   merge_down<8, N>(v, lane, (lane & 32) == 0);  // lanes 0-15 descending, 32-47 ascending
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const u64 o = xr64<32>(v[i], lane);
+    const Key o = xr64<32>(v[i], lane);
     v[i] = o > v[i] ? o : v[i];
   }
   merge_down<8, N>(v, lane, true);

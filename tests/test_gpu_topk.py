@@ -195,3 +195,31 @@ def test_stage1_repeats_bit_for_bit(gpu_lib, M, n, noise):
         else:
             assert torch.equal(sub_idx, first[0]), f"run {it}: {int((sub_idx != first[0]).sum())} ids differ"
             assert torch.equal(sub_sc, first[1]), f"run {it}: scores differ"
+
+
+@pytest.mark.parametrize("M,n,k,sign", [(3, 64, 16, -1.0), (70, 100, 32, -1.0), (70, 100, 9, 1.0), (2, 1024, 16, -1.0)])
+def test_equal_scores_of_either_sign_order_by_index(gpu_lib, M, n, k, sign):
+    """All keys of a codebook are one vector, along the query or against it:
+    every score is the same number, positive or negative, so the k best are
+    the k lowest indices (lax.top_k's order).  Exact: equal scores have equal
+    bits, whatever their sign."""
+    L = _lib.lib()
+    H, half, score = 2, 64, _lib.MPL_F16
+    g = torch.Generator().manual_seed(n + k)
+    base = torch.randn((1, H, 2, half), generator=g)
+    q = base.repeat(M, 1, 1, 1).cuda()
+    keys = (sign * base[0])[:, :, None, :].repeat(1, 1, n, 1).contiguous().cuda()
+    packed = torch.empty(L.mpl_packed_keys_bytes(H, n, half, score), dtype=torch.uint8, device="cuda")
+    st = _lib.stream_ptr(q.device)
+    _lib.check(L.mpl_pack_keys(_lib.ptr(keys), H, n, half, score, None, _lib.ptr(packed), st), "pack")
+    T_dev = torch.full((1,), 10.0, device="cuda")
+    wsb = L.mpl_score_topk_workspace_bytes(M, H, n, half, k)
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+    ids = torch.full((M, H, 2, k), -7, dtype=torch.int32, device="cuda")
+    sc = torch.empty((M, H, 2, k), dtype=torch.float32, device="cuda")
+    _lib.check(L.mpl_score_topk(_lib.ptr(q), _lib.MPL_Q_RAW, None, _lib.ptr(packed), M, H, n, half, k, score,
+                                _lib.ptr(T_dev), None, None, _lib.ptr(ws), wsb, _lib.ptr(ids), _lib.ptr(sc), st),
+               "topk")
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(ids.cpu().numpy(), np.broadcast_to(np.arange(k), (M, H, 2, k)))
+    assert bool(((sc * sign) > 0).all())
