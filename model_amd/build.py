@@ -33,6 +33,11 @@ FLAGS = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 
+# Flags of single files, beyond FLAGS.  score_sort.hip: no IEEE mode and no NaN
+# handling of min / max, whose canonicalisation would add an instruction to
+# every key (the file turns NaN scores into -inf before they become keys).
+FILE_FLAGS = {"score_sort.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
+
 
 def hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
@@ -58,7 +63,7 @@ def _compile(src: str, cc: str) -> str:
     if src.endswith(".cpp"):
         cmd = [host_cxx(), *HOST_FLAGS, "-c", src, "-o", obj]
     else:
-        cmd = [cc, *FLAGS, "-c", src, "-o", obj]
+        cmd = [cc, *FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")

@@ -2,8 +2,11 @@
 // top-k (memory.py:149-164), then stage-2 top-k over the k*k candidates and
 // the routing softmax (memory.py:167-178).
 //
-// Stage 1 (score_topk_kernel).  A workgroup of two waves handles one
-// codebook hc = h*2 + c and one split of its n sub-keys; each wave owns 32
+// Stage 1 takes one of two kernels (make_clean_plan): score_sort_kernel
+// (score_sort.hip) sorts every block's scores in registers, for short key
+// ranges a wave; score_topk_kernel, here, filters them by thresholds, for long
+// ones and with routing noise.  Of score_topk_kernel, a workgroup of two waves
+// handles one codebook hc = h*2 + c and one split of its n sub-keys; each wave owns 32
 // queries.  The queries are normalised in registers (or read normalised) and
 // held as the MFMA B operand; each block of 32 keys is one chain of 32x32
 // MFMAs (keys = A operand).  Key blocks reach the waves one of two ways,
@@ -52,6 +55,7 @@
 #include "common.h"
 #include "layout.h"
 #include "mfma.h"
+#include "score_stage1.h"
 #include "topk.h"
 #include "wsum.h"
 
@@ -69,30 +73,11 @@ constexpr int kNoiseCand = MPL_NOISE_CAND;  // the same with routing noise
 #define MPL_SCORE_THREADS 128
 #endif
 constexpr int kScoreThreads = MPL_SCORE_THREADS;  // waves per workgroup x 64
-constexpr int kQueriesPerWave = 32;
 constexpr int kQueriesPerGroup = kQueriesPerWave * (kScoreThreads / 64);
 #ifndef MPL_MAX_SPLITS
 #define MPL_MAX_SPLITS 64
 #endif
 constexpr int kMaxSplits = MPL_MAX_SPLITS;
-
-struct ScoreParams {
-  const void* q_hat;    // [M, HC, half]: normalised in the scoring type (mode 0) or raw fp32
-  const float* q_len;   // [M, HC] or null (mode 0 input)
-  float* out_qlen;      // [M, HC] or null (mode 2 output)
-  int query_mode;       // MPL_Q_NORMALIZED / MPL_Q_RAW / MPL_Q_RAW_SCALED
-  const uint4* packed;  // packed keys
-  const float* gumbel;  // [M, HC, n] or null
-  const float* T;           // device scalar: the clamped temperature
-  const float* noise_coef;  // device scalar routing_noise * noise_scale (read with noise only)
-  int noise_vec;  // gumbel rows 16-byte aligned (base aligned, n % 4 == 0)
-  int64_t M;
-  int HC, n, half, k, nblk, splits, blk_per_split;
-  int pass1_blocks;  // blocks of each split scanned by the bound pass
-  float* out_sel;    // [splits, HC, k, M] (null without noise: equals clean)
-  float* out_clean;  // [splits, HC, k, M]
-  int* out_idx;      // [splits, HC, k, M]
-};
 
 // Per-lane selection state of the stage-1 kernel.  Candidates are appended
 // to the lane's column of two LDS arrays of [waves][entries][64] words
@@ -328,57 +313,6 @@ __device__ __forceinline__ float kth_of_pair16(const float* own, int par, int k)
   return from_orderable(r);
 }
 
-// The wave's MFMA query operand: lane l holds query row my_q (= the wave's
-// first query + l % 32), dims 16c + 8*(l/32) + [0,8) of chunk c (fp16; the
-// fp32 tile's map for fp32), and ql, the row's length factor (1 without
-// query_scale / q_len).  Rows out of range (!valid) are zeros.  With
-// write_qlen, mode RAW_SCALED also stores ql to out_qlen.
-template <typename T, int NCH>
-__device__ __forceinline__ void query_operand(const ScoreParams& p, int hc, int64_t my_q, bool valid, int lane,
-                                              bool write_qlen, typename Mfma<T>::Op (&qop)[NCH], float& ql) {
-  const int par = lane >> 5;
-  ql = 1.f;
-  if (p.query_mode == MPL_Q_NORMALIZED) {
-    const T* qrow = (const T*)p.q_hat + (valid ? (my_q * p.HC + hc) * (int64_t)p.half : 0);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) qop[c] = Mfma<T>::load_q(qrow, valid, p.half, c, lane);
-    if (p.q_len != nullptr) ql = p.q_len[(valid ? my_q : 0) * p.HC + hc];
-  } else {
-    // Raw fp32 queries, normalised here (memory.py:30-31, 136-137): the
-    // lane pair holds the row's 2*NCH*8 dims, so one half-swap completes
-    // the sum of squares.
-    const float* qrow = (const float*)p.q_hat + (valid ? (my_q * p.HC + hc) * (int64_t)p.half : 0);
-    float x[NCH][Mfma<T>::kQElems];
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) Mfma<T>::load_q_raw(qrow, valid, p.half, c, lane, x[c], ss);
-    float a = ss, b = ss;
-    half_swap(a, b);
-    const float tot = ss + (par ? a : b) + 1e-6f;
-    const float rn = 1.0f / sqrtf(tot);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) qop[c] = Mfma<T>::scale_q(x[c], rn);
-    if (p.query_mode == MPL_Q_RAW_SCALED) {
-      ql = sqrtf(tot) / sqrtf((float)p.half);
-      if (p.out_qlen != nullptr && valid && write_qlen && par == 0) p.out_qlen[my_q * p.HC + hc] = ql;
-    }
-  }
-}
-
-// Short splits (SB = 4 or 8 blocks at most, no noise: the decode-sized
-// plans): the workgroup copies all of the split's key blocks into LDS by LDS
-// DMA at kernel start, each wave scores every block once from there, and
-// both passes read the scores from the MFMA accumulators instead of
-// reloading and re-scoring.  The key tiles lie in the candidate arrays,
-// which the select pass takes over after a barrier; the arrays hold 64
-// entries per lane, so SB = 4 needs no overflow check inside the pass and
-// SB = 8 one per block from the fifth on.  SB = 0: the streaming passes.
-constexpr int kShortCand = 64;
-template <typename T, int HP>
-constexpr bool short_fits(int sb) {
-  return sb * KeyPack<T>::vectors_per_lane(HP) * kWave * 16 <= 2 * (kScoreThreads / kWave) * kShortCand * kWave * 4;
-}
-
 // Minimum waves per SIMD the compiler allocates registers for: the noisy
 // fp16 selection with k <= 16 is held to two (its 38.5 KB of LDS per
 // workgroup allows two per SIMD; without the bound it took 259 registers and
@@ -388,7 +322,7 @@ constexpr int stage1_min_waves() {
   return (NOISE && KMAX == 16 && sizeof(T) == 2) ? 2 : 1;
 }
 
-template <typename T, int HP, bool NOISE, int KMAX, bool DIRECT, int SB>
+template <typename T, int HP, bool NOISE, int KMAX, bool DIRECT>
 __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())) void score_topk_kernel(
     ScoreParams p) {
   constexpr int VPL = KeyPack<T>::vectors_per_lane(HP);  // 16-B vectors per lane per block
@@ -396,15 +330,13 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
   constexpr int NCH = VPL * OPV;                         // MFMA chunks per block
   constexpr int TILE = VPL * kWave;                      // uint4 per key block
   constexpr int WAVES = kScoreThreads / kWave;
-  constexpr bool SHORT = SB > 0;
   typedef typename Mfma<T>::Op Op;
-  static_assert(!SHORT || (!NOISE && short_fits<T, HP>(SB)), "short splits: no noise, key tiles fit the arrays");
 
   // with noise the buffer holds two arrays of 22 entries per lane (clean
   // score and index), so that with the key tiles a workgroup takes 38.5 KB of
   // LDS and two fit each SIMD
-  constexpr int CAND = SHORT ? kShortCand : (NOISE ? kNoiseCand : kCand);
-  __shared__ uint4 tile0[DIRECT || SHORT ? 1 : TILE], tile1[DIRECT || SHORT ? 1 : TILE];  // the LDS path's key tiles
+  constexpr int CAND = NOISE ? kNoiseCand : kCand;
+  __shared__ uint4 tile0[DIRECT ? 1 : TILE], tile1[DIRECT ? 1 : TILE];  // the LDS path's key tiles
   __shared__ float cscore[WAVES * CAND * kWave];
   __shared__ uint32_t cindex[WAVES * CAND * kWave];
 
@@ -448,19 +380,6 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
                                        0);
     }
   };
-  // Short splits: tile j of the split in the candidate arrays (TPA tiles in
-  // each), requested here for all blocks b_begin + j (clamped to the split,
-  // so past its end a block repeats the last one) before the query, so that
-  // keys and query arrive in one memory round trip.
-  constexpr int TPA = (int)(sizeof(cscore) / (TILE * sizeof(uint4)));
-  auto short_tile = [&](int j) __attribute__((always_inline)) {
-    return j < TPA ? (uint4*)cscore + j * TILE : (uint4*)cindex + (j - TPA) * TILE;
-  };
-  if constexpr (SHORT) {
-#pragma unroll
-    for (int j = 0; j < SB; ++j) dma(short_tile(j), min(b_begin + j, b_end - 1));
-  }
-
   Op qop[NCH];
   float ql;
   query_operand<T, NCH>(p, hc, my_q, valid, lane, split == 0, qop, ql);
@@ -596,40 +515,9 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
     sweep_lds_on(tile0, tile1, bb, be, body);
   };
 
-  f32x16 sacc[SHORT ? SB : 1];
-  if constexpr (SHORT) {
-    // every wave's DMA (and its query loads) landed: the scores of the
-    // split's blocks (past the split's end a block repeats the last one,
-    // which the passes skip or which leaves the maxima as they are)
-    wait_vmcnt_le<0>();
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < SB; ++j) {
-      const uint4* tl = short_tile(j);
-      f32x16 x = f32x16{};
-#pragma unroll
-      for (int v = 0; v < VPL; ++v) {
-        const uint4 u = tl[v * kWave + lane];
-#pragma unroll
-        for (int e = 0; e < OPV; ++e) x = Mfma<T>::mma(Mfma<T>::from_vec(u, e), qop[v * OPV + e], x);
-      }
-      sacc[SHORT ? j : 0] = x;
-    }
-    // both waves' tile reads are done before the select pass writes
-    // candidates over the tiles
-    __syncthreads();
-  }
   auto sweep = [&](int bb, int be, auto&& body) __attribute__((always_inline)) {
-    if constexpr (SHORT) {
-      const GVec g{};
-      auto no_issue = [](int) {};
-#pragma unroll
-      for (int j = 0; j < SB; ++j) body((bb + j) * 32, sacc[SHORT ? j : 0], g, j < be - bb, no_issue);
-    } else if constexpr (DIRECT) {
-      sweep_direct(bb, be, body);
-    } else {
-      sweep_lds(bb, be, body);
-    }
+    if constexpr (DIRECT) sweep_direct(bb, be, body);
+    else sweep_lds(bb, be, body);
   };
 
   // Selection values of the lane's 16 keys of a block (padded keys -inf);
@@ -677,9 +565,8 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
     for (int r = 0; r < 16; ++r) {
       issue_for(r, issue);
       const float v = raw ? c[r] : sv[r];
-      // Past the end (!active) c holds a block of the split again (the last
-      // one, or with SHORT a block pass 2 scans anyway), so its maxima are
-      // still scores of this split's keys: no test of `active` is needed.
+      // Past the end (!active) c holds the split's last block again, whose
+      // maxima are still scores of this split's keys: no test of `active`.
       ma[r] = max(ma[r], __float_as_int(v));
     }
     (void)active;
@@ -690,7 +577,7 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
   // two tiles laid over the candidate arrays (unused until the select pass,
   // which starts after every DMA has landed and both waves are past the
   // last tile read).  The select pass keeps register-loaded keys.
-  constexpr bool LDS_BOUND = DIRECT && !SHORT && !NOISE && sizeof(cscore) >= TILE * sizeof(uint4) &&
+  constexpr bool LDS_BOUND = DIRECT && !NOISE && sizeof(cscore) >= TILE * sizeof(uint4) &&
                              sizeof(cindex) >= TILE * sizeof(uint4);
   if constexpr (LDS_BOUND) {
     sweep_lds_on((uint4*)cscore, (uint4*)cindex, b_begin, p1_end, bound_body);
@@ -746,41 +633,20 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
       st.off += (active && x > st.thr) ? kEntryBytes : 0u;
     }
   };
-  if constexpr (SHORT) {
-    // block j adds at most 16 entries to the 16 * j before it: from the
-    // block that could overflow on, a check flushes above CAND - 16
-    const uint32_t flush16 = lane0 + (uint32_t)(CAND - 16) * kEntryBytes;
-    auto no_issue = [](int) {};
+  sweep(b_begin, b_end, [&](int kb, const f32x16& c, const GVec& g, bool active, auto&& issue)
+                            __attribute__((always_inline)) {
+    float sv[16];
+    lane_scores(kb, c, g, sv);
 #pragma unroll
-    for (int j = 0; j < SB; ++j) {
-      const int kb = (b_begin + j) * 32;
-      const bool active = j < b_end - b_begin;
-      if (16 * (j + 1) > CAND && active && __ballot(st.off > flush16) != 0) {
+    for (int q = 0; q < 2; ++q) {
+      // the flush check before each group of 8 leaves 8 free entries
+      if (active && __ballot(st.off > flush_at) != 0) {
         flush_lane<true, KMAX, NOISE, CAND>(st, cscore, cindex, grow, coef, lane0, valid, p.k, base_thr, par);
         flushed = true;
       }
-      float sv[16];
-      const GVec g{};
-      lane_scores(kb, sacc[SHORT ? j : 0], g, sv);
-      append8(kb, sacc[SHORT ? j : 0], sv, active, 0, no_issue);
-      append8(kb, sacc[SHORT ? j : 0], sv, active, 1, no_issue);
+      append8(kb, c, sv, active, q, issue);
     }
-  } else {
-    sweep(b_begin, b_end, [&](int kb, const f32x16& c, const GVec& g, bool active, auto&& issue)
-                              __attribute__((always_inline)) {
-      float sv[16];
-      lane_scores(kb, c, g, sv);
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        // the flush check before each group of 8 leaves 8 free entries
-        if (active && __ballot(st.off > flush_at) != 0) {
-          flush_lane<true, KMAX, NOISE, CAND>(st, cscore, cindex, grow, coef, lane0, valid, p.k, base_thr, par);
-          flushed = true;
-        }
-        append8(kb, c, sv, active, q, issue);
-      }
-    });
-  }
+  });
   {
     const int cnt_own = (int)((st.off - lane0) / kEntryBytes);
     float ca = __int_as_float(cnt_own), cb = ca;
@@ -1688,40 +1554,104 @@ __global__ __launch_bounds__(1024) void pair_decode_read_k16(PairParams p, ReadP
 }
 
 // ---------------------------------------------------------------- host side
+static int padded_half(int half, int score_dtype) {
+  return score_dtype == MPL_F16 ? KeyPack<_Float16>::padded_half(half) : KeyPack<float>::padded_half(half);
+}
+
 struct Plan {
   int splits, blk_per_split, nblk, kmax, pass1_blocks;
   int64_t qblocks;
+  bool sort;  // stage 1 by sorting (score_sort.hip)
 };
 
-// Workgroups a launch should reach before the key range is split (two waves
-// each: two waves per SIMD of the 256 CUs, so that one wave's selection work
-// overlaps the other's MFMAs).
-#ifndef MPL_SCORE_TARGET_WGS
-#define MPL_SCORE_TARGET_WGS 1024
-#endif
-// The bound pass scans min(blocks, max(MIN, blocks / DIV)) blocks of a split.
-#ifndef MPL_PASS1_MIN
-#define MPL_PASS1_MIN 16
-#endif
-#ifndef MPL_PASS1_DIV
-#define MPL_PASS1_DIV 8
-#endif
+// Blocks of a split that the thresholds' bound pass scans.  Without noise a
+// few: its scores cost more than the flushes that a looser bound brings
+// (8,192 tokens, n = 512: 36.0 us of stage 1 from 4 blocks, 37.7 from 16;
+// 4,096 tokens, n = 8,192, 128 blocks a split: 126.5 from 8, 129.7 from 16).
+// With noise a flush also reads the noise of its candidates again (8,192
+// tokens, n = 512: 79.7 us from 16 blocks, 86.4 from 4).
+static int bound_blocks(int blk, bool noise) {
+  return std::min(blk, noise ? std::max(16, blk / 8) : std::max(4, blk / 16));
+}
 
+// The most splits a plan takes: up to two waves a SIMD (1,024 workgroups of
+// two), so a workspace holds at most that many lists.
+static int most_splits(int64_t M, int H, int nblk) {
+  return (int)std::min<int64_t>(std::min(nblk, kMaxSplits), cdiv(1024, cdiv(M, kQueriesPerGroup) * 2 * H));
+}
+
+// The plan of a call with routing noise: as many splits as keep the waves at
+// one a SIMD.  A wave's fixed work (its queries, the bound, the flushes and
+// the pair merge, 20 us and more) counts once a split, so splits past that
+// only add it (4,001 tokens, n = 300: 38.6 us of stage 1 unsplit, 50.7 in
+// two, 58.8 in three; 2,000 tokens, n = 128, fp32: 42.2 / 39.5 / 38.3 / 66.1
+// in one to four).
 static Plan make_plan(int64_t M, int H, int n, int k) {
   Plan pl;
   pl.nblk = (int)cdiv(n, 32);
   pl.qblocks = cdiv(M, kQueriesPerGroup);
-  const int64_t base = pl.qblocks * 2 * H;
-  int64_t s = cdiv(MPL_SCORE_TARGET_WGS, base);
-  s = s < 1 ? 1 : s;
-  s = s > kMaxSplits ? kMaxSplits : s;
-  s = s > pl.nblk ? pl.nblk : s;
+  int64_t s = 1024 / (cdiv(M, kQueriesPerWave) * 2 * H);
+  s = std::max<int64_t>(1, std::min<int64_t>(s, most_splits(M, H, pl.nblk)));
   pl.blk_per_split = (int)cdiv(pl.nblk, s);
   pl.splits = (int)cdiv(pl.nblk, pl.blk_per_split);
   pl.kmax = k <= 16 ? 16 : 32;
-  const int p1 = pl.blk_per_split / MPL_PASS1_DIV;
-  pl.pass1_blocks = std::min(pl.blk_per_split, std::max(MPL_PASS1_MIN, p1));
+  pl.pass1_blocks = bound_blocks(pl.blk_per_split, true);
+  pl.sort = false;
   return pl;
+}
+
+// The plan of a call without routing noise: stage 1 by sorting
+// (score_sort.hip) or by thresholds (score_topk_kernel), and into how many
+// splits, whichever this model of the time (us) makes shortest.  W is the
+// waves per SIMD (of 1,024), a wave being 32 queries of one codebook and one
+// split.
+//   sort:       7 + 2 W + c blocks max(1, ceil(W)), c = 0.7 (from W > 1 on,
+//               where the VALU is full, 0.75 for stage 1 alone and 1.0 with
+//               stage 2 behind it, which the sort slows by 4 us in 47), 1.6 c
+//               for k > 16;
+//   thresholds: 16 + 4 W + blocks (0.49 + 0.13 W) for W <= 1, rounds of two
+//               waves a SIMD beyond, each 23 + 0.82 blocks;
+//   fp32 scoring adds its MFMAs to both, 1.8 us a block at half = 128 (twice
+//   to the thresholds' bound pass); splits add their lists' traffic and what
+//   stage 2 takes to combine them.
+// Measured on MI355X (lookup, us, sort / thresholds at their best splits):
+// 64 tokens, n = 4,096: 16.9 / 19.2; 150: 20.4 / 24.1; 600 tokens, n = 512:
+// 17.3 / 20.2; 8,192 tokens, n = 128: 44.7 / 50.8; 2,048 tokens, n = 2,048:
+// 46.7 / 52.3; the other way 8,192 tokens, n = 512: 81.9 / 77.7 and 4,096
+// tokens, n = 4,096: 122.7 / 105.0.  The training step's clean lists (8,192
+// tokens, n = 512, stage 1 alone, beside the noise fill): 883 us a step by
+// sorting, 885 by thresholds from 16 blocks and 909 from 4.
+static Plan make_clean_plan(int64_t M, int H, int n, int k, int score_dtype, int HP, bool pair) {
+  Plan best = make_plan(M, H, n, k);
+  const int nblk = best.nblk;
+  const double base = (double)(cdiv(M, kQueriesPerWave) * 2 * H) / 1024.0;
+  const double mf = score_dtype == MPL_F32 ? 1.8 * HP / 128 : 0.0;
+  double tbest = 1e300;
+  int last = 0;
+  const int most = most_splits(M, H, nblk);
+  for (int s = 1; s <= most; ++s) {
+    const int blk = (int)cdiv(nblk, s);
+    if (blk == last) continue;  // the same splits as before
+    last = blk;
+    const int S = (int)cdiv(nblk, blk);
+    const double W = base * S;
+    double lists = 0.0;
+    if (S > 1) lists = (S <= 4 ? 2 : S <= 8 ? 5 : S <= 32 ? 3 : 7) + (double)M * 2 * H * k * 16 * S * 2e-7;
+    if (S > 1 && k != 16) lists += 0.7 * S;  // pair_kernel takes them one after the other
+    const double c = (W <= 1 ? 0.7 : pair ? 1.0 : 0.75) * (k > 16 ? 1.6 : 1.0);
+    const double t_sort = 7 + 2 * std::min(W, 2.0) + blk * (c + mf) * std::max(1.0, std::ceil(W)) + lists;
+    const double p1 = mf * bound_blocks(blk, false);  // the bound pass scores its blocks again
+    const double t_thr = (W <= 1 ? 16 + 4 * W + blk * (0.49 + 0.13 * W + mf) + p1
+                                 : std::ceil(W / 2) * (23 + blk * (0.82 + 2 * mf) + 2 * p1)) + lists;
+    if (std::min(t_sort, t_thr) < tbest) {
+      tbest = std::min(t_sort, t_thr);
+      best.sort = t_sort <= t_thr;
+      best.splits = S;
+      best.blk_per_split = blk;
+      best.pass1_blocks = bound_blocks(blk, false);
+    }
+  }
+  return best;
 }
 
 // Decode plans (score_topk_decode): M <= kDecodeMaxQ tokens and k <= 16,
@@ -1736,6 +1666,7 @@ static Plan make_decode_plan(int n) {
   pl.splits = (int)cdiv(pl.nblk, pl.blk_per_split);
   pl.kmax = 16;
   pl.pass1_blocks = 0;
+  pl.sort = false;
   return pl;
 }
 
@@ -1767,19 +1698,7 @@ constexpr bool direct_keys() {
 template <typename T, int HP, bool NOISE, int KMAX>
 static void launch_stage1(const ScoreParams& sp, int64_t blocks, hipStream_t s) {
   constexpr bool D = direct_keys<T, HP, NOISE, KMAX>();
-  if constexpr (!NOISE && short_fits<T, HP>(4)) {
-    if (sp.blk_per_split <= 4) {
-      score_topk_kernel<T, HP, NOISE, KMAX, false, 4><<<(unsigned)blocks, kScoreThreads, 0, s>>>(sp);
-      return;
-    }
-  }
-  if constexpr (!NOISE && short_fits<T, HP>(8)) {
-    if (sp.blk_per_split <= 8) {
-      score_topk_kernel<T, HP, NOISE, KMAX, false, 8><<<(unsigned)blocks, kScoreThreads, 0, s>>>(sp);
-      return;
-    }
-  }
-  score_topk_kernel<T, HP, NOISE, KMAX, D, 0><<<(unsigned)blocks, kScoreThreads, 0, s>>>(sp);
+  score_topk_kernel<T, HP, NOISE, KMAX, D><<<(unsigned)blocks, kScoreThreads, 0, s>>>(sp);
 }
 
 template <int HP>
@@ -1848,23 +1767,25 @@ static size_t topk_extra_bytes(const Plan& pl, int64_t M, int H, int k) {
   return (pl.splits > 1 && k != 16) ? (size_t)M * H * k * 3 * 4 : 0;
 }
 
-// The sizes cover every plan a call of these shapes may take (the decode
-// plan depends on the scoring type and noise, which the size query lacks).
+// The sizes cover every plan a call of these shapes may take (the plans
+// depend on the scoring type and noise, which the size queries lack).
 extern "C" size_t mpl_score_select_workspace_bytes(int64_t M, int H, int n, int half, int k) {
-  (void)half;
   if (M <= 0 || H <= 0 || n <= 0 || k <= 0) return 0;
   size_t need = ws_bytes(make_plan(M, H, n, k), M, H, k, true);
+  for (int dt : {MPL_F16, MPL_F32})
+    need = std::max(need, ws_bytes(make_clean_plan(M, H, n, k, dt, padded_half(half, dt), true), M, H, k, false));
   if (decode_shape(M, k)) need = std::max(need, ws_bytes(make_decode_plan(n), M, H, k, false));
   return need;
 }
 
 extern "C" size_t mpl_score_topk_workspace_bytes(int64_t M, int H, int n, int half, int k) {
-  (void)half;
   if (M <= 0 || H <= 0 || n <= 0 || k <= 0) return 0;
   auto need = [&](const Plan& pl, bool noise) {
     return (ws_bytes(pl, M, H, k, noise) + 255) / 256 * 256 + topk_extra_bytes(pl, M, H, k);
   };
   size_t b = need(make_plan(M, H, n, k), true);
+  for (int dt : {MPL_F16, MPL_F32})
+    b = std::max(b, need(make_clean_plan(M, H, n, k, dt, padded_half(half, dt), false), false));
   if (decode_shape(M, k)) b = std::max(b, need(make_decode_plan(n), false));
   return b;
 }
@@ -2005,7 +1926,9 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
               MPL_EINVAL, "%s: bad query_mode %d", who, query_mode);
   const bool noise = gumbel != nullptr;
   const bool decode = !noise && score_dtype == MPL_F16 && decode_shape(M, k);
-  const Plan pl = decode ? make_decode_plan(n) : make_plan(M, H, n, k);
+  const int HP = padded_half(half, score_dtype);
+  const Plan pl = decode ? make_decode_plan(n) : noise ? make_plan(M, H, n, k)
+                                       : make_clean_plan(M, H, n, k, score_dtype, HP, pair);
   const size_t sel_need = ws_bytes(pl, M, H, k, noise);
   const size_t extra = pair ? 0 : topk_extra_bytes(pl, M, H, k);
   const size_t extra_at = (sel_need + 255) / 256 * 256;
@@ -2046,9 +1969,9 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
     sp.out_idx = (int*)(w + part);
     sp.out_sel = noise ? w + 2 * part : nullptr;
   }
-  const int HP = score_dtype == MPL_F16 ? KeyPack<_Float16>::padded_half(half) : KeyPack<float>::padded_half(half);
   const int64_t blocks = pl.qblocks * pl.splits * HC;
   int rc = decode ? dispatch_decode(sp, blocks, HP, s)
+           : pl.sort ? launch_score_sort(sp, score_dtype, HP, pl.kmax, s)
                   : dispatch_stage1(sp, blocks, score_dtype, HP, noise, pl.kmax, s);
   if (rc) {
     set_error("%s: unsupported padded half %d", who, HP);

@@ -84,6 +84,28 @@ __device__ __forceinline__ void sort8(Key* c, float* p) {
 #undef MPL_CE
 }
 
+// Sorts 16 keys descending (Green's 60-comparator network, checked over all
+// 2^16 zero-one inputs).
+__device__ __forceinline__ void sort16(Key* c) {
+#define MPL_CE(i, j)                              \
+  {                                               \
+    const Key hi_ = __builtin_fmax(c[i], c[j]);   \
+    c[j] = __builtin_fmin(c[i], c[j]);            \
+    c[i] = hi_;                                   \
+  }
+  MPL_CE(0, 1) MPL_CE(2, 3) MPL_CE(4, 5) MPL_CE(6, 7) MPL_CE(8, 9) MPL_CE(10, 11) MPL_CE(12, 13) MPL_CE(14, 15)
+  MPL_CE(0, 2) MPL_CE(1, 3) MPL_CE(4, 6) MPL_CE(5, 7) MPL_CE(8, 10) MPL_CE(9, 11) MPL_CE(12, 14) MPL_CE(13, 15)
+  MPL_CE(0, 4) MPL_CE(1, 5) MPL_CE(2, 6) MPL_CE(3, 7) MPL_CE(8, 12) MPL_CE(9, 13) MPL_CE(10, 14) MPL_CE(11, 15)
+  MPL_CE(0, 8) MPL_CE(1, 9) MPL_CE(2, 10) MPL_CE(3, 11) MPL_CE(4, 12) MPL_CE(5, 13) MPL_CE(6, 14) MPL_CE(7, 15)
+  MPL_CE(5, 10) MPL_CE(6, 9) MPL_CE(3, 12) MPL_CE(13, 14) MPL_CE(4, 8) MPL_CE(7, 11) MPL_CE(1, 2)
+  MPL_CE(1, 4) MPL_CE(7, 13) MPL_CE(2, 8) MPL_CE(11, 14)
+  MPL_CE(2, 4) MPL_CE(5, 6) MPL_CE(9, 10) MPL_CE(11, 13) MPL_CE(3, 8) MPL_CE(7, 12)
+  MPL_CE(6, 8) MPL_CE(10, 12) MPL_CE(3, 5) MPL_CE(7, 9)
+  MPL_CE(3, 4) MPL_CE(5, 6) MPL_CE(7, 8) MPL_CE(9, 10) MPL_CE(11, 12)
+  MPL_CE(6, 7) MPL_CE(8, 9)
+#undef MPL_CE
+}
+
 template <int KMAX, bool PAY>
 struct TopList {
   Key key[KMAX];

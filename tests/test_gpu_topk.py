@@ -223,3 +223,52 @@ def test_equal_scores_of_either_sign_order_by_index(gpu_lib, M, n, k, sign):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(ids.cpu().numpy(), np.broadcast_to(np.arange(k), (M, H, 2, k)))
     assert bool(((sc * sign) > 0).all())
+
+
+@pytest.mark.parametrize("M,n,half,k,score,bad", [
+    (5, 33, 16, 16, _lib.MPL_F16, False),     # two key blocks, one key in the second; a few query rows
+    (31, 32, 32, 1, _lib.MPL_F16, False),     # one block, k = 1
+    (33, 47, 64, 17, _lib.MPL_F16, False),    # k > 16 on a ragged block, a second query tile of one row
+    (64, 512, 128, 16, _lib.MPL_F16, True),   # split lists; NaN queries and a NaN key
+    (1, 700, 8, 16, _lib.MPL_F32, False),     # fp32, one query, ragged splits
+    (40, 300, 20, 32, _lib.MPL_F32, True),    # fp32 width off the pack sizes, k = 32
+    (700, 100, 128, 9, _lib.MPL_F32, False),  # k < 16 with fp32 MFMAs over several blocks
+    (3000, 300, 64, 16, _lib.MPL_F16, True),  # unsplit, ten blocks a wave
+])
+def test_sorted_stage1_equals_thresholds(gpu_lib, M, n, half, k, score, bad):
+    """Stage 1 by sorting (no noise) against stage 1 by thresholds, which a
+    call with noise takes: with zero noise, coefficient 0 and T = 1 both order
+    the same scores, so ids and scores are equal bit for bit, rows and keys of
+    NaN (never selected, id -1 where a list stays short) included."""
+    L = _lib.lib()
+    H = 2
+    g = torch.Generator().manual_seed(M + n + half)
+    q = torch.randn((M, H, 2, half), generator=g)
+    keys = torch.randn((H, 2, n, half), generator=g)
+    keys[:, :, 1::7] = keys[:, :, :1]  # repeated keys: exact ties
+    if bad:
+        q[1::3, 0, 1] = float("nan")
+        keys[1, 0, n // 2] = float("nan")
+    q, keys = q.cuda(), keys.contiguous().cuda()
+    packed = torch.empty(L.mpl_packed_keys_bytes(H, n, half, score), dtype=torch.uint8, device="cuda")
+    st = _lib.stream_ptr(q.device)
+    _lib.check(L.mpl_pack_keys(_lib.ptr(keys), H, n, half, score, None, _lib.ptr(packed), st), "pack")
+    one = torch.ones(1, device="cuda")
+    zero = torch.zeros(1, device="cuda")
+    no_noise = torch.zeros((M, H, 2, n), device="cuda")
+    wsb = L.mpl_score_topk_workspace_bytes(M, H, n, half, k)
+    got = []
+    for gum in (None, no_noise):
+        ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+        ids = torch.full((M, H, 2, k), -7, dtype=torch.int32, device="cuda")
+        sc = torch.full((M, H, 2, k), 7.0, device="cuda")
+        _lib.check(L.mpl_score_topk(_lib.ptr(q), _lib.MPL_Q_RAW, None, _lib.ptr(packed), M, H, n, half, k, score,
+                                    _lib.ptr(one), _lib.ptr(gum), _lib.ptr(zero if gum is not None else None),
+                                    _lib.ptr(ws), wsb, _lib.ptr(ids), _lib.ptr(sc), st), "topk")
+        torch.cuda.synchronize()
+        got.append((ids.cpu().numpy(), sc.cpu().numpy()))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    assert bad or int(got[0][0].min()) >= 0
+    if bad:
+        assert (got[0][0][1::3, 0, 1] == -1).all()
