@@ -31,6 +31,28 @@ __global__ __launch_bounds__(kGatherThreads) void gather_wsum_kernel(
   acc.store(out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
 }
 
+// Rows of any other number of 16-byte vectors up to 64 (WsumAny).
+template <typename V, bool NT>
+__global__ __launch_bounds__(kGatherThreads) void gather_wsum_any(
+    const V* __restrict__ values, int64_t N, int VR, const int32_t* __restrict__ slots,
+    const float* __restrict__ weights, int64_t M, int R, int shuffle, float* __restrict__ out) {
+  const int64_t m = (int64_t)blockIdx.x * (kGatherThreads / kWave) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (m >= M) return;
+  WsumAny<V, NT> acc(VR, lane);
+  for (int r0 = 0; r0 < R; r0 += kWave) {
+    const int rr = r0 + lane;
+    const bool in = rr < R;
+    int sl = slots[m * R + (in ? rr : 0)];  // unconditional (clamped) loads
+    float ww = weights[m * R + (in ? rr : 0)];
+    if (shuffle) sl = (int)(((int64_t)sl + N / 2 + 1) % N);
+    sl = in ? (int)min(max((int64_t)sl, (int64_t)0), N - 1) : 0;  // out-of-range ids read the nearest row
+    ww = in ? ww : 0.f;
+    acc.add_chunk((const uint4*)values, sl, ww, min(kWave, R - r0));
+  }
+  acc.store(out + m * (int64_t)VR * WsumAny<V, NT>::VE, lane);
+}
+
 // Any d: one thread per (token, column).
 template <typename V>
 __global__ __launch_bounds__(256) void gather_wsum_generic(const V* __restrict__ values, int64_t N, int d,
@@ -70,6 +92,11 @@ static int gather_impl(const V* values, int64_t N, int d, const int32_t* slots, 
       MPL_G(1) MPL_G(2) MPL_G(4) MPL_G(8) MPL_G(16) MPL_G(32) MPL_G(64) MPL_G(128) MPL_G(256)
 #undef MPL_G
       default: break;
+    }
+    if (VR <= kWave) {
+      if (nt) gather_wsum_any<V, true><<<blocks, kGatherThreads, 0, s>>>(values, N, VR, slots, w, M, R, shuffle, out);
+      else gather_wsum_any<V, false><<<blocks, kGatherThreads, 0, s>>>(values, N, VR, slots, w, M, R, shuffle, out);
+      return check_launch("mpl_gather_wsum");
     }
   }
   gather_wsum_generic<V><<<(unsigned)cdiv(M * d, 256), 256, 0, s>>>(values, N, d, slots, w, M, R, shuffle, out);

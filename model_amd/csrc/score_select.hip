@@ -40,12 +40,12 @@
 // the per-split lists are merged (merge_splits_k16 reduces eight lists per
 // 16-lane row at a time) before stage 2.
 //
-// Stage 2 (pair_kernel_k16 for k = 16, pair_kernel<G> otherwise).  A row of
+// Stage 2 (pair_kernel_k16 for k <= 16, pair_kernel_k32 otherwise).  A row of
 // 16 lanes (k <= 16) or a group of 32 per (token, head) merges the lists of
 // both codebooks, walks the k*k candidate grid as sorted row lists keyed by
 // (select sum desc, flat index rank_a*k + rank_b asc) as memory.py:171, and
 // finishes with the softmax of the clean slot scores (memory.py:178).  The
-// k = 16 kernel exchanges values with DPP and ds_swizzle only.
+// k <= 16 kernels exchange values with DPP and ds_swizzle only.
 #include <limits.h>
 
 #include <algorithm>
@@ -877,15 +877,15 @@ struct PairParams {
   float* weights;      // [M, H, k]
 };
 
-// A group of G lanes per (token, head).  Per codebook, the S split lists are
+// A group of 32 lanes per (token, head), for k > 16.  Per codebook, the S split lists are
 // combined with cross-lane bitonic merges (lane r ends with the rank-r
 // entry).  The k*k candidates of memory.py:167-171 are then merged row by
 // row as lists keyed (select sum, flat index rank_a*k + rank_b): row i holds
 // k/(i+1) candidates that can still reach the top k, and the rows with a
 // single such candidate (i >= k/2) form one more sorted list.  The softmax
 // of memory.py:178 runs across the group.
-template <int G>
-__global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
+__global__ __launch_bounds__(256) void pair_kernel_k32(PairParams p) {
+  constexpr int G = 32;
   const int lane = threadIdx.x & 63;
   const int r = lane % G;
   const int base = lane - r;
@@ -983,19 +983,23 @@ __global__ __launch_bounds__(256) void pair_kernel(PairParams p) {
   }
 }
 
-// pair_kernel for k == 16: the same algorithm on 16-lane rows with DPP /
-// swizzle exchanges (no LDS traffic) and compile-time row broadcasts; split
-// lists are loaded four at a time so their loads overlap.
+// The same for k <= 16 on 16-lane rows, with DPP / swizzle exchanges (no LDS
+// traffic) and compile-time row broadcasts.  KT is k where it is known (16),
+// or 0: lists of p.k < 16 entries then leave the lanes past them empty, and
+// the 16 x 16 grid below covers the k x k candidates (a pair (i, j) with
+// (i+1)(j+1) > 16 has more than k better ones).
 // The pair stage of one (token, head) on a 16-lane row, from the two
 // codebooks' final lists (lane r holds rank r of lk[c], clean score lc[c]):
 // memory.py:167-175.  Writes slots, flat indices and routing weights of a
 // live row.
 // The lane's slot id (in [0, n*n)) and weight are also returned in slot_out
 // and w_out, for a value read fused behind the pair stage.
+template <int KT>
 __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&lk)[2], const float (&lc)[2],
                                               bool live, int64_t mh, int lane, int r, int& slot_out,
                                               float& w_out) {
   constexpr int K = 16;
+  const int k = KT ? KT : p.k;
   const bool a_ok = has_key(lk[0]), b_ok = has_key(lk[1]);
   const float a_sel = a_ok ? key_score(lk[0]) : -INFINITY;
   const float b_sel = b_ok ? key_score(lk[1]) : -INFINITY;
@@ -1014,7 +1018,7 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&l
 #define MPL_PAIR_ROW(I)                                                                                 \
   {                                                                                                     \
     const float ai = g16::bcastf<I>(a_sel), aic = g16::bcastf<I>(a_cl), aik = g16::bcastf<I>(aok);    \
-    L[I] = (r < K / (I + 1) && aik != 0.f && b_ok) ? make_key(ai + b_sel, I * K + r) : kNoKey;           \
+    L[I] = (r < K / (I + 1) && aik != 0.f && b_ok) ? make_key(ai + b_sel, I * k + r) : kNoKey;           \
     P[I] = aic + b_cl;                                                                                  \
   }
   MPL_PAIR_ROW(0) MPL_PAIR_ROW(1) MPL_PAIR_ROW(2) MPL_PAIR_ROW(3) MPL_PAIR_ROW(4) MPL_PAIR_ROW(5)
@@ -1026,7 +1030,7 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&l
     const float ar = __uint_as_float(g16::shl8(__float_as_uint(a_sel)));
     const float arc = __uint_as_float(g16::shl8(__float_as_uint(a_cl)));
     const float ark = __uint_as_float(g16::shl8(__float_as_uint(aok)));
-    L[8] = (r < 8 && ark != 0.f && b0_ok) ? make_key(ar + b0, (8 + r) * K) : kNoKey;
+    L[8] = (r < 8 && ark != 0.f && b0_ok) ? make_key(ar + b0, (8 + r) * k) : kNoKey;
     P[8] = arc + b0c;
   }
 #pragma unroll
@@ -1038,21 +1042,22 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&l
   const Key acc = L[0];
   const float pay = P[0];
 
-  // lane r holds the rank-r slot
-  const int flat = has_key(acc) ? key_index(acc) : 0;
+  // lane r < k holds the rank-r slot
+  const bool mine = has_key(acc) && r < k;
+  const int flat = mine ? key_index(acc) : 0;
   const int base = lane - r;
-  int ia = __shfl(a_id, base + flat / K);
-  int ib = __shfl(b_id, base + flat % K);
+  int ia = __shfl(a_id, base + flat / k);
+  int ib = __shfl(b_id, base + flat % k);
   ia = (ia >= 0 && ia < p.n) ? ia : 0;  // ids come from keys < n; guards non-finite inputs
   ib = (ib >= 0 && ib < p.n) ? ib : 0;
-  const float sc = has_key(acc) ? pay : -INFINITY;
+  const float sc = mine ? pay : -INFINITY;
   const float mx = g16::rmax(sc);
-  const float e = has_key(acc) ? expf(sc - mx) : 0.f;
+  const float e = mine ? expf(sc - mx) : 0.f;
   const float sum = g16::rsum(e);
   slot_out = ia * p.n + ib;
   w_out = e / sum;
-  if (live) {
-    const int64_t ob = mh * K + r;
+  if (live && r < k) {
+    const int64_t ob = mh * k + r;
     p.slots[ob] = slot_out;
     p.flat_idx[ob] = flat;
     p.weights[ob] = w_out;
@@ -1061,9 +1066,11 @@ __device__ __forceinline__ void pair_tail_k16(const PairParams& p, const Key (&l
 
 // The two codebooks' final lists of row mh (lane r gets rank r of lk[c] and
 // its clean score lc[c]): one split list loaded, or S lists merged.
+template <int KT>
 __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, int64_t mh, int r, Key (&lk)[2],
                                                float (&lc)[2]) {
-  constexpr int K = 16;
+  const int k = KT ? KT : p.k;
+  const bool in = live && r < k;
   const int64_t m = live ? mh / p.H : 0;
   const int h = live ? (int)(mh % p.H) : 0;
   const int HC = 2 * p.H;
@@ -1075,7 +1082,7 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
   // merge at all.
   int64_t o0[2];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) o0[c] = ((int64_t)m * HC + 2 * h + c) * K + r;
+  for (int c = 0; c < 2; ++c) o0[c] = ((int64_t)m * HC + 2 * h + c) * k + (r < k ? r : 0);
   if (p.S == 1) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -1083,11 +1090,11 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
       float sl[1] = {lsel[o0[c]]}, cc[1] = {p.clean[o0[c]]};
       pin_loaded(id, sl, cc);
       lc[c] = cc[0];
-      lk[c] = (live && id[0] >= 0) ? make_key(sl[0], id[0]) : kNoKey;
+      lk[c] = (in && id[0] >= 0) ? make_key(sl[0], id[0]) : kNoKey;
     }
   } else {
     constexpr int B = 8;
-    const int64_t sstride = p.M * HC * K;
+    const int64_t sstride = p.M * HC * k;
     for (int s0 = 0; s0 < p.S; s0 += B) {
       int id[2][B];
       float sl[2][B], cc[2][B];
@@ -1107,7 +1114,7 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
 #pragma unroll
         for (int t = 0; t < B; ++t) {
           if (s0 + t < p.S) {  // uniform
-            const Key kk = (live && id[c][t] >= 0) ? make_key(sl[c][t], id[c][t]) : kNoKey;
+            const Key kk = (in && id[c][t] >= 0) ? make_key(sl[c][t], id[c][t]) : kNoKey;
             if (s0 + t == 0) {
               lk[c] = kk;
               lc[c] = cc[c][t];
@@ -1119,13 +1126,14 @@ __device__ __forceinline__ void pair_lists_k16(const PairParams& p, bool live, i
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c)
-      if (live) {
+      if (in) {
         p.sub_idx[o0[c]] = has_key(lk[c]) ? key_index(lk[c]) : -1;
         p.sub_scores[o0[c]] = has_key(lk[c]) ? lc[c] : -INFINITY;
       }
   }
 }
 
+template <int KT>
 __global__ __launch_bounds__(256) void pair_kernel_k16(PairParams p) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 15;
@@ -1133,10 +1141,10 @@ __global__ __launch_bounds__(256) void pair_kernel_k16(PairParams p) {
   const bool live = mh < p.M * p.H;  // dead rows still join the exchanges
   Key lk[2];
   float lc[2];
-  pair_lists_k16(p, live, mh, r, lk, lc);
+  pair_lists_k16<KT>(p, live, mh, r, lk, lc);
   int slot;
   float w;
-  pair_tail_k16(p, lk, lc, live, mh, lane, r, slot, w);
+  pair_tail_k16<KT>(p, lk, lc, live, mh, lane, r, slot, w);
 }
 
 // The value read of a fused lookup (memory.py:179-193): values [n*n, VR*16
@@ -1160,10 +1168,10 @@ __global__ __launch_bounds__(256) void pair_read_k16(PairParams p, ReadParams rp
   const bool live = mh < p.M * 4;  // H = 4: a wave is live or dead as a whole
   Key lk[2];
   float lc[2];
-  pair_lists_k16(p, live, mh, r, lk, lc);
+  pair_lists_k16<16>(p, live, mh, r, lk, lc);
   int slot;
   float w;
-  pair_tail_k16(p, lk, lc, live, mh, lane, r, slot, w);
+  pair_tail_k16<16>(p, lk, lc, live, mh, lane, r, slot, w);
   if (!live) return;
   const int64_t m = mh >> 2;
   const int64_t N = (int64_t)p.n * p.n;
@@ -1173,31 +1181,59 @@ __global__ __launch_bounds__(256) void pair_read_k16(PairParams p, ReadParams rp
   acc.store(rp.out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
 }
 
-// Split lists are reduced eight at a time before stage 2 (k == 16 only).
+// pair_read_k16 for k < 16, or rows of any number VR <= 64 of 16-byte vectors
+// (WsumAny): the token's H*k rows move from lanes h*16 + r to lanes h*k + r
+// first, the order gather_wsum reads them in.
+template <typename V, bool NT>
+__global__ __launch_bounds__(256) void pair_read_any(PairParams p, ReadParams rp, int VR) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15;
+  const int64_t mh = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
+  const bool live = mh < p.M * 4;  // H = 4: a wave is live or dead as a whole
+  Key lk[2];
+  float lc[2];
+  pair_lists_k16<0>(p, live, mh, r, lk, lc);
+  int slot;
+  float w;
+  pair_tail_k16<0>(p, lk, lc, live, mh, lane, r, slot, w);
+  if (!live) return;
+  const int64_t m = mh >> 2;
+  const int64_t N = (int64_t)p.n * p.n;
+  if (rp.shuffle) slot = (int)(((int64_t)slot + N / 2 + 1) % N);
+  const int src = lane < 4 * p.k ? lane / p.k * 16 + lane % p.k : lane;
+  slot = __shfl(slot, src);
+  w = __shfl(w, src);
+  WsumAny<V, NT> acc(VR, lane);
+  acc.add_chunk((const uint4*)rp.values, slot, w, 4 * p.k);
+  acc.store(rp.out + m * (int64_t)VR * Vec16<V>::kElems, lane);
+}
+
+// Split lists are reduced eight at a time before stage 2 (k <= 16).
 constexpr int kMergeChunk = 8;
 
-// Split-list reduction for k == 16: 16-lane row (s2, m, hc) merges lists
+// Split-list reduction for k <= 16: 16-lane row (s2, m, hc) merges lists
 // s2*8 .. s2*8+7 of (m, hc) (loaded four at a time) into list s2.
 struct MergeParams {
   const float* sel;  // null without noise (equals clean)
   const float* clean;
   const int* idx;
   int64_t rows;  // M * HC
-  int S, S2;
+  int S, S2, k;
   float* out_sel;
   float* out_clean;
   int* out_idx;
 };
 
 __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
-  constexpr int K = 16;
+  const int k = p.k;
   const int r = threadIdx.x & 15;
+  const int rk = r < k ? r : 0;
   const int64_t g = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
   const bool live = g < p.rows * p.S2;  // dead rows still join the exchanges
   const int64_t row = live ? g % p.rows : 0;
   const int s2 = live ? (int)(g / p.rows) : 0;
   const float* lsel = p.sel != nullptr ? p.sel : p.clean;
-  const int64_t sstride = p.rows * K;
+  const int64_t sstride = p.rows * k;
   // All lists of the chunk are requested before the first merge (one memory
   // round trip).  Lists past p.S read the last list again and enter as empty
   // keys; an empty key's payload is never output, so it is passed as loaded.
@@ -1206,7 +1242,7 @@ __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
 #pragma unroll
   for (int t = 0; t < kMergeChunk; ++t) {
     const int s = min(s2 * kMergeChunk + t, p.S - 1);  // clamped, unconditional
-    const int64_t o = (int64_t)s * sstride + row * K + r;
+    const int64_t o = (int64_t)s * sstride + row * k + rk;
     id[t] = p.idx[o];
     sl[t] = lsel[o];
     cc[t] = p.clean[o];
@@ -1217,7 +1253,7 @@ __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
 #pragma unroll
   for (int t = 0; t < kMergeChunk; ++t) {
     const bool in = s2 * kMergeChunk + t < p.S;  // uniform per row
-    const Key kk = (in && id[t] >= 0) ? make_key(sl[t], id[t]) : kNoKey;
+    const Key kk = (in && r < k && id[t] >= 0) ? make_key(sl[t], id[t]) : kNoKey;
     if (t == 0) {
       acc = kk;
       pay = cc[t];
@@ -1225,8 +1261,8 @@ __global__ __launch_bounds__(256) void merge_splits_k16(MergeParams p) {
       g16::merge(acc, pay, kk, cc[t], r);
     }
   }
-  if (live) {
-    const int64_t o = ((int64_t)s2 * p.rows + row) * K + r;
+  if (live && r < k) {
+    const int64_t o = ((int64_t)s2 * p.rows + row) * k + r;
     p.out_idx[o] = has_key(acc) ? key_index(acc) : -1;
     p.out_clean[o] = has_key(acc) ? pay : -INFINITY;
     if (p.out_sel != nullptr) p.out_sel[o] = has_key(acc) ? key_score(acc) : -INFINITY;
@@ -1297,7 +1333,7 @@ __global__ __launch_bounds__(256) void pair_wide_k16(PairParams p) {
     const float lc[2] = {spay[0][r], spay[8][r]};
     int slot;
     float w;
-    pair_tail_k16(p, lk, lc, true, mh, lane, r, slot, w);
+    pair_tail_k16<16>(p, lk, lc, true, mh, lane, r, slot, w);
   }
 }
 
@@ -1368,7 +1404,7 @@ __global__ __launch_bounds__(1024) void pair_wide_read_k16(PairParams p, ReadPar
     const float lc[2] = {spay[h][0][r], spay[h][8][r]};
     int slot;
     float w;
-    pair_tail_k16(p, lk, lc, true, mh, lane, r, slot, w);
+    pair_tail_k16<16>(p, lk, lc, true, mh, lane, r, slot, w);
     srow_slot[h * K + r] = slot;
     srow_w[h * K + r] = w;
   }
@@ -1637,7 +1673,7 @@ static Plan make_clean_plan(int64_t M, int H, int n, int k, int score_dtype, int
     const double W = base * S;
     double lists = 0.0;
     if (S > 1) lists = (S <= 4 ? 2 : S <= 8 ? 5 : S <= 32 ? 3 : 7) + (double)M * 2 * H * k * 16 * S * 2e-7;
-    if (S > 1 && k != 16) lists += 0.7 * S;  // pair_kernel takes them one after the other
+    if (S > 1 && k > 16) lists += 0.7 * S;  // pair_kernel_k32 takes them one after the other
     const double c = (W <= 1 ? 0.7 : pair ? 1.0 : 0.75) * (k > 16 ? 1.6 : 1.0);
     const double t_sort = 7 + 2 * std::min(W, 2.0) + blk * (c + mf) * std::max(1.0, std::ceil(W)) + lists;
     const double p1 = mf * bound_blocks(blk, false);  // the bound pass scores its blocks again
@@ -1671,11 +1707,11 @@ static Plan make_decode_plan(int n) {
 }
 
 // Workspace: the select scores with noise; per-split lists when split, and
-// for k == 16 the lists of each reduction level (8 lists into one) until at
+// for k <= 16 the lists of each reduction level (8 lists into one) until at
 // most 8 remain for stage 2.
 static int reduced_total(const Plan& pl, int k) {
   int tot = 0;
-  for (int S = pl.splits; k == 16 && S > kMergeChunk; S = (int)cdiv(S, kMergeChunk)) tot += (int)cdiv(S, kMergeChunk);
+  for (int S = pl.splits; k <= 16 && S > kMergeChunk; S = (int)cdiv(S, kMergeChunk)) tot += (int)cdiv(S, kMergeChunk);
   return tot;
 }
 
@@ -1761,10 +1797,10 @@ static int dispatch_stage1(const ScoreParams& sp, int64_t blocks, int score_dtyp
 using namespace mpl;
 
 // Scratch of the stage-1-only call beyond the selection's: with several
-// splits and k != 16 the lists are combined by the pair kernel, whose slot
+// splits and k > 16 the lists are combined by the pair kernel, whose slot
 // outputs (flat_idx, slots, weights) then go to scratch.
 static size_t topk_extra_bytes(const Plan& pl, int64_t M, int H, int k) {
-  return (pl.splits > 1 && k != 16) ? (size_t)M * H * k * 3 * 4 : 0;
+  return (pl.splits > 1 && k > 16) ? (size_t)M * H * k * 3 * 4 : 0;
 }
 
 // The sizes cover every plan a call of these shapes may take (the plans
@@ -1804,7 +1840,7 @@ struct LookupRead {
 
 static bool launch_pair_read(const LookupRead& lr, const PairParams& pp, unsigned grid, hipStream_t s) {
   const int esz = lr.dtype == MPL_F16 ? 2 : 4;
-  if (pp.H != 4 || pp.k != 16 || (lr.d * esz) % 16 != 0 || ((uintptr_t)lr.values % 16) != 0 ||
+  if (pp.H != 4 || pp.k > 16 || (lr.d * esz) % 16 != 0 || ((uintptr_t)lr.values % 16) != 0 ||
       ((uintptr_t)lr.out % 16) != 0)
     return false;
   ReadParams rp;
@@ -1821,13 +1857,23 @@ static bool launch_pair_read(const LookupRead& lr, const PairParams& pp, unsigne
       pair_read_k16<V, vr, false><<<grid, 256, 0, s>>>(pp, rp);     \
     return true;                                                    \
   }
-  if (lr.dtype == MPL_F16) {
-    MPL_PR(_Float16, 16) MPL_PR(_Float16, 32) MPL_PR(_Float16, 64)
-  } else {
-    MPL_PR(float, 32) MPL_PR(float, 64)
+  if (pp.k == 16) {
+    if (lr.dtype == MPL_F16) {
+      MPL_PR(_Float16, 16) MPL_PR(_Float16, 32) MPL_PR(_Float16, 64)
+    } else {
+      MPL_PR(float, 32) MPL_PR(float, 64)
+    }
   }
 #undef MPL_PR
-  return false;
+  if (VR > kWave) return false;
+  if (lr.dtype == MPL_F16) {
+    if (nt) pair_read_any<_Float16, true><<<grid, 256, 0, s>>>(pp, rp, VR);
+    else pair_read_any<_Float16, false><<<grid, 256, 0, s>>>(pp, rp, VR);
+  } else {
+    if (nt) pair_read_any<float, true><<<grid, 256, 0, s>>>(pp, rp, VR);
+    else pair_read_any<float, false><<<grid, 256, 0, s>>>(pp, rp, VR);
+  }
+  return true;
 }
 
 // The value read fused into pair_wide_k16 (pair_wide_read_k16): same shape
@@ -2010,7 +2056,7 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
     return check_launch("mpl_score_select(stage 2)");
   }
   float* r = w + (noise ? 3 : 2) * part;
-  while (k == 16 && pp.S > kMergeChunk) {
+  while (k <= 16 && pp.S > kMergeChunk) {
     const int S2 = (int)cdiv(pp.S, kMergeChunk);
     const size_t part2 = per * S2;
     MergeParams mp;
@@ -2020,6 +2066,7 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
     mp.rows = M * HC;
     mp.S = pp.S;
     mp.S2 = S2;
+    mp.k = k;
     mp.out_clean = r;
     mp.out_idx = (int*)(r + part2);
     mp.out_sel = noise ? r + 2 * part2 : nullptr;
@@ -2033,7 +2080,7 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
     r += (noise ? 3 : 2) * part2;
   }
   if (!pair && pp.S == 1) return MPL_OK;  // stage 1 wrote sub_idx / sub_scores
-  if (!pair && k == 16) {
+  if (!pair && k <= 16) {
     // the last reduction level writes the single list straight to the outputs
     MergeParams mp;
     mp.sel = pp.sel;
@@ -2042,28 +2089,28 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
     mp.rows = M * HC;
     mp.S = pp.S;
     mp.S2 = 1;
+    mp.k = k;
     mp.out_clean = sub_scores;
     mp.out_idx = sub_idx;
     mp.out_sel = nullptr;
     merge_splits_k16<<<(unsigned)cdiv(mp.rows * 16, 256), 256, 0, s>>>(mp);
     return check_launch("mpl_score_topk(split merge)");
   }
-  if (!pair) {  // k != 16 with splits: the pair kernel combines them; its slot outputs go to scratch
+  if (!pair) {  // k > 16 with splits: the pair kernel combines them; its slot outputs go to scratch
     char* x = (char*)workspace + extra_at;
     const size_t mhk = (size_t)M * H * k;
     pp.flat_idx = (int32_t*)x;
     pp.slots = (int32_t*)(x + mhk * 4);
     pp.weights = (float*)(x + mhk * 8);
   }
-  const int G = k <= 16 ? 16 : 32;
-  const unsigned g2 = (unsigned)cdiv(M * H * G, 256);
-  if (k == 16 && read != nullptr && launch_pair_read(*read, pp, g2, s)) {
+  const unsigned g2 = (unsigned)cdiv(M * H * (k <= 16 ? 16 : 32), 256);
+  if (k <= 16 && read != nullptr && launch_pair_read(*read, pp, g2, s)) {
     *read_done = true;
     return check_launch("mpl_lookup(stage 2 + value read)");
   }
-  if (k == 16) pair_kernel_k16<<<g2, 256, 0, s>>>(pp);
-  else if (G == 16) pair_kernel<16><<<g2, 256, 0, s>>>(pp);
-  else pair_kernel<32><<<g2, 256, 0, s>>>(pp);
+  if (k == 16) pair_kernel_k16<16><<<g2, 256, 0, s>>>(pp);
+  else if (k < 16) pair_kernel_k16<0><<<g2, 256, 0, s>>>(pp);
+  else pair_kernel_k32<<<g2, 256, 0, s>>>(pp);
   return check_launch(pair ? "mpl_score_select(stage 2)" : "mpl_score_topk(split lists)");
 }
 

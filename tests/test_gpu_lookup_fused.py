@@ -76,6 +76,40 @@ def test_lookup_equals_select_then_gather(gpu_lib, M, H, n, d_key, d, k, vdt, sh
     assert bool((got["slots"] >= 0).all()) and bool((got["slots"] < n * n).all())
 
 
+@pytest.mark.parametrize("M,H,n,d_key,d,k,vdt,shuffle", [
+    (301, 4, 100, 64, 192, 8, torch.float16, 1),     # 24 vectors a row: two rows a load, 16 lanes idle
+    (77, 4, 64, 64, 24, 5, torch.float16, 0),        # 3 vectors: 21 rows a load, 20 rows a token
+    (50, 4, 64, 64, 8, 1, torch.float16, 0),         # one vector a row, k = 1
+    (200, 4, 64, 32, 100, 16, torch.float32, 0),     # 25 fp32 vectors
+    (130, 4, 300, 128, 512, 7, torch.float16, 0),    # 64 vectors, k < 16
+    (65, 4, 64, 64, 132, 16, torch.float32, 1),      # 33 vectors: one row a load, 31 lanes idle
+    (9, 4, 3000, 64, 192, 16, torch.float16, 0),     # more than 8 split lists, no fused width: two launches
+    (9, 4, 3000, 64, 192, 4, torch.float16, 1),      # more than 8 split lists of k < 16
+    (40, 2, 200, 64, 48, 11, torch.float32, 0),      # H = 2: two launches
+    (30, 8, 200, 64, 520, 8, torch.float16, 0),      # 65 vectors: a thread per column
+])
+def test_any_row_width_and_k(gpu_lib, M, H, n, d_key, d, k, vdt, shuffle):
+    """Row widths of any number of 16-byte vectors and k < 16: the lookup
+    equals the two-launch path bit for bit, and both equal the sum of the
+    selected rows in 64 bits within the rounding of H*k fp32 terms (each
+    product and sum rounds to 2^-24 relative: H*k * 2^-24 * sum |w v|)."""
+    ref, got = _run(M, H, n, d_key, d, k, vdt, shuffle, seed=M + n)
+    for name in ref:
+        assert torch.equal(ref[name], got[name]), name
+    N = n * n
+    g = torch.Generator(device="cuda").manual_seed(M + n)  # _run's values
+    torch.randn((M, H, 2, d_key // 2), generator=g, device="cuda")
+    torch.randn((H, 2, n, d_key // 2), generator=g, device="cuda")
+    values = (torch.randn((N, d), generator=g, device="cuda") * 0.02).to(vdt).double()
+    s = got["slots"].long().reshape(M, -1)
+    assert bool((s >= 0).all()) and bool((s < N).all())
+    terms = got["weights"].double().reshape(M, -1, 1) * values[(s + N // 2 + 1) % N if shuffle else s]
+    bound = H * k * 2.0 ** -24 * terms.abs().sum(1) + 1e-12
+    assert bool(((got["out"].double() - terms.sum(1)).abs() <= bound).all())
+    torch.testing.assert_close(got["weights"].double().sum(-1), torch.ones((M, H), device="cuda").double(),
+                               rtol=0, atol=k * 2.0 ** -22)
+
+
 def test_lookup_zero_tokens_and_errors(gpu_lib):
     L = _lib.lib()
     s = torch.cuda.current_stream().cuda_stream
