@@ -610,6 +610,37 @@ int mpl_rows_linear_pair(const float* x, const float* ln_scale, const float* ln_
                          int K, int N1, int N2, float* out1, float* out2, void* stream);
 
 /*
+ * Up to three dense layers of the same rows in one launch, for many rows (the
+ * backbone over whole sequences, model.py:87-126: the query / key / value
+ * projections, the router and gate, the feed-forward and output layers):
+ *   a = x [rows, K] fp32, LayerNorm and x_mul as in mpl_rows_linear;
+ *   outs[i] [rows, out_pitches[i]] = act_i(a . weights[i] + biases[i]) (+ residual)
+ * on fp32 MFMA tiles.  weights (const float*[count], each [K, widths[i]] or
+ * [widths[i], K] by weight_layout, 16-byte aligned), biases (const
+ * float*[count], entries may be NULL), widths (int[count], multiples of 4),
+ * activations (int[count]), outs (float*[count]) and out_pitches
+ * (int64_t[count], in floats, >= width) are host tables read by the call.
+ * residual [rows, widths[0]] (or NULL) goes with count = 1; the output may be
+ * the residual but not x or x_mul.  K is a multiple of 4; x, x_mul, ln_scale
+ * and ln_bias are 16-byte aligned.  Deterministic; a layer's result does not
+ * depend on the others of the launch.
+ */
+int mpl_dense_layers(const float* x, const float* x_mul, const float* ln_scale, const float* ln_bias, float ln_eps,
+                     int count, const void* weights, int weight_layout, const void* biases, const void* widths,
+                     const void* activations, const float* residual, const void* outs, const void* out_pitches,
+                     int64_t rows, int K, void* stream);
+
+/*
+ * Causal self-attention over whole sequences, forward (model.py:88-95 outside
+ * decode mode): out [batch, T, heads, head_dim] = softmax over s <= t of
+ * (scale * q_t) . k_s, times v_s, from qkv [batch, T, 3, heads, head_dim]
+ * fp32 (biases added, 16-byte aligned), in fp32 with an online softmax.
+ * head_dim is 32, 64 or 128 (else MPL_EUNSUPPORTED); batch * heads <= 65535.
+ */
+int mpl_causal_attention(const float* qkv, int64_t batch, int T, int heads, int head_dim, float scale, float* out,
+                         void* stream);
+
+/*
  * The output layer of a decode step (model.py:125-126): logits [rows, V] =
  * LayerNorm(x) . emb^T (ln_final, then embed.attend), x [rows, d], emb
  * [V, d] (x, ln_scale, ln_bias and emb 16-byte aligned), LayerNorm as in mpl_rows_linear (mean and

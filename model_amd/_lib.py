@@ -79,6 +79,8 @@ SIGNATURES = {
                                          _I64, _I, _P, _P]),
     "mpl_decode_embed": (_I, [_P, _I64, _P, _I64, _I, _P, _P, _I64, _P, _P]),
     "mpl_rows_linear": (_I, [_P, _P, _P, _P, _F, _P, _I, _P, _I, _P, _I64, _I, _I, _P, _P]),
+    "mpl_dense_layers": (_I, [_P, _P, _P, _P, _F, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I64, _I, _P]),
+    "mpl_causal_attention": (_I, [_P, _I64, _I, _I, _I, _F, _P, _P]),
     "mpl_vocab_logits": (_I, [_P, _P, _P, _F, _P, _I64, _I, _I64, _P, _P]),
     "mpl_rows_linear_pair": (_I, [_P, _P, _P, _F, _P, _P, _I, _I, _I64, _I, _I, _I, _P, _P, _P]),
     "mpl_balance_state_bytes": (_SZ, [_I64, _I]),

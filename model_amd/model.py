@@ -29,6 +29,7 @@ concatenated once per parameter version, not on every step.
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 import math
 from typing import Any, Dict, List, Optional, Tuple
@@ -175,6 +176,79 @@ def rows_linear_pair(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
         P(bias), _ACT[act1], _ACT[act2], rows, K, n1, n2, P(out1), P(out2), _lib.stream_ptr(x.device)),
         "mpl_rows_linear_pair")
     return out1, out2
+
+
+def dense_layers(x: torch.Tensor, layers, *, ln: Optional[Dict[str, torch.Tensor]] = None, eps: float = LN_EPS,
+                 x_mul: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None,
+                 out_in: bool = False, joined: bool = False) -> List[torch.Tensor]:
+    """mpl_dense_layers: up to three dense layers of the same rows x [rows, K]
+    fp32 in one launch, for many rows: ``layers`` holds (weight, bias or None,
+    activation or None) each, the weight a Dense kernel [K, ...] or, with
+    ``out_in``, a table [N, K].  ``joined`` puts the outputs side by side in
+    one [rows, sum of widths] tensor (the list then holds it alone)."""
+    from . import _lib
+
+    rows, K = x.shape
+    ws = [w.reshape(-1, K) if out_in else w.reshape(K, -1) for w, _, _ in layers]
+    bs = [None if b is None else b.reshape(-1) for _, b, _ in layers]
+    widths = [w.shape[0] if out_in else w.shape[1] for w in ws]
+    ts = [x, *ws] + [t for t in (*bs, x_mul, residual) if t is not None]
+    if ln is not None:
+        ts += [ln["scale"], ln["bias"]]
+    for t in ts:
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.device != x.device:
+            raise ValueError("dense_layers: operands must be contiguous fp32 on one device")
+    if x.device.type != "cuda":
+        raise ValueError("dense_layers runs on the GPU only (libmpl.so)")
+    if (any(b is not None and b.numel() != n for b, n in zip(bs, widths))
+            or (x_mul is not None and x_mul.shape != x.shape)
+            or (residual is not None and (len(ws) != 1 or residual.shape != (rows, widths[0])))
+            or (ln is not None and (ln["scale"].numel() != K or ln["bias"].numel() != K))):
+        raise ValueError(f"dense_layers: operand shapes do not fit x {tuple(x.shape)} and widths {widths}")
+    n = len(ws)
+    if joined:
+        outs = [torch.empty((rows, sum(widths)), dtype=torch.float32, device=x.device)]
+        ptrs = [outs[0].data_ptr() + 4 * sum(widths[:i]) for i in range(n)]
+        pitches = [sum(widths)] * n
+    else:
+        outs = [torch.empty((rows, w), dtype=torch.float32, device=x.device) for w in widths]
+        ptrs, pitches = [o.data_ptr() for o in outs], widths
+    P = _lib.ptr
+    table = lambda kind, v: ctypes.cast((kind * n)(*v), ctypes.c_void_p)  # noqa: E731
+    _lib.check(_lib.lib().mpl_dense_layers(
+        P(x), P(x_mul), P(None if ln is None else ln["scale"]), P(None if ln is None else ln["bias"]), float(eps), n,
+        table(ctypes.c_void_p, [w.data_ptr() for w in ws]), _lib.MPL_W_OUT_IN if out_in else _lib.MPL_W_IN_OUT,
+        table(ctypes.c_void_p, [P(b) for b in bs]), table(ctypes.c_int, widths),
+        table(ctypes.c_int, [_ACT[act] for _, _, act in layers]), P(residual), table(ctypes.c_void_p, ptrs),
+        table(ctypes.c_int64, pitches), rows, K, _lib.stream_ptr(x.device)), "mpl_dense_layers")
+    return outs
+
+
+def causal_attention(qkv: torch.Tensor, heads: int, scale: float) -> torch.Tensor:
+    """mpl_causal_attention: qkv [B, T, 3 * heads * hd] fp32 (query, key and
+    value projections, biases added) -> [B, T, heads * hd]."""
+    from . import _lib
+
+    B, T, w = qkv.shape
+    hd = w // (3 * heads)
+    if (w != 3 * heads * hd or qkv.dtype != torch.float32 or not qkv.is_contiguous()
+            or qkv.device.type != "cuda"):
+        raise ValueError(f"causal_attention: qkv {tuple(qkv.shape)} must be contiguous fp32 [B, T, 3 * heads * hd] "
+                         "on the GPU")
+    out = torch.empty((B, T, heads * hd), dtype=torch.float32, device=qkv.device)
+    _lib.check(_lib.lib().mpl_causal_attention(qkv.data_ptr(), B, T, heads, hd, float(scale), out.data_ptr(),
+                                               _lib.stream_ptr(qkv.device)), "mpl_causal_attention")
+    return out
+
+
+def _plain_inference() -> bool:
+    """Whether torch ops run here as they are written: no gradient mode, and
+    none of the modes that replace, record or transform them (forward-mode
+    AD, functorch, tracing, compilation, autocast, dispatch modes)."""
+    return (not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled()
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
 
 
 def decode_attention(qkv: torch.Tensor, positions: torch.Tensor, layer_cache: Dict[str, torch.Tensor], heads: int,
@@ -463,6 +537,67 @@ class MemoryPoolLM:
                 logits = F.linear(_ln(x, lf), emb)[:, None]
         return logits, _LazyMerged(layer_aux)
 
+    def _fused_forward_ok(self, p, tokens) -> bool:
+        """Whether _forward_gpu computes this call: plain inference on the
+        GPU with fp32 parameters whose widths the fused kernels take."""
+        cfg = self.cfg
+        d, H = cfg.d_model, cfg.n_heads
+        if (not tokens.is_cuda or type(tokens) is not torch.Tensor or tokens.numel() == 0 or not _plain_inference()
+                or d % 4 or d % H or d // H not in (32, 64, 128) or tokens.shape[0] * H > 65535
+                or tokens.numel() > 65535 * 64 or cfg.pool_heads * cfg.d_key % 4 or cfg.d_value % 4):
+            return False
+
+        def plain(t):
+            if isinstance(t, dict):
+                return all(plain(v) for v in t.values())
+            return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_contiguous()
+                    and t.device == tokens.device and t.data_ptr() % 16 == 0)
+
+        names = ["ln_final"]
+        for i in range(cfg.n_layers):
+            mem = self.pool is not None and i in cfg.memory_layers
+            names += [f"ln_attn_{i}", f"attn_{i}", f"ln_ffn_{i}"]
+            names += [f"ffn_in_{i}", f"ffn_out_{i}"] if not mem or cfg.memory_ffn else []
+            names += [f"router_{i}", f"mem_gate_{i}", f"mem_out_{i}"] if mem else []
+        emb, pe = p["embed"]["embedding"], p["pos_embed"]
+        return plain(emb) and plain(pe) and emb.shape[0] % 4 == 0 and all(plain(p[nm]) for nm in names)
+
+    def _forward_gpu(self, p, tokens, pool_off, noise_scale, shuffle_pool, rngs):
+        """The general path of apply() for plain inference over whole
+        sequences, as library launches: the layer norms, biases, activations
+        and residual adds inside the dense layers (mpl_dense_layers), and the
+        attention one launch without score matrix, mask or transposed copies
+        (mpl_causal_attention)."""
+        cfg = self.cfg
+        B, T = tokens.shape
+        d, H = cfg.d_model, cfg.n_heads
+        emb = p["embed"]["embedding"]
+        x = (emb[tokens] + p["pos_embed"][None, :T]).reshape(B * T, d)
+        layer_aux = []
+        for i in range(cfg.n_layers):
+            pa = p[f"attn_{i}"]
+            qkv, = dense_layers(x, [(pa[nm]["kernel"], pa[nm]["bias"], None) for nm in ("query", "key", "value")],
+                                ln=p[f"ln_attn_{i}"], joined=True)
+            a = causal_attention(qkv.reshape(B, T, 3 * d), H, (d // H) ** -0.5)
+            x, = dense_layers(a.reshape(B * T, d), [(pa["out"]["kernel"], pa["out"]["bias"], None)], residual=x)
+            ln = p[f"ln_ffn_{i}"]
+            mem_layer = self.pool is not None and i in cfg.memory_layers
+            x_in = x
+            if not mem_layer or cfg.memory_ffn:
+                fi, fo = p[f"ffn_in_{i}"], p[f"ffn_out_{i}"]
+                hid, = dense_layers(x_in, [(fi["kernel"], fi["bias"], "gelu_tanh")], ln=ln)
+                x, = dense_layers(hid, [(fo["kernel"], fo["bias"], None)], residual=x)
+            if mem_layer and not pool_off:
+                r, g, mo = p[f"router_{i}"], p[f"mem_gate_{i}"], p[f"mem_out_{i}"]
+                q, gate = dense_layers(x_in, [(r["kernel"], r["bias"], None), (g["kernel"], g["bias"], "silu")], ln=ln)
+                mem, aux = self.pool.apply({"params": p["pool"]}, q.reshape(B, T, cfg.pool_heads, cfg.d_key),
+                                           noise_scale=noise_scale, shuffle_reads=shuffle_pool, rngs=rngs)
+                x, = dense_layers(mem.reshape(B * T, cfg.d_value), [(mo["kernel"], mo["bias"], None)], x_mul=gate,
+                                  residual=x)
+                layer_aux.append(aux)
+        logits = F.linear(_ln(x, p["ln_final"]), emb)
+        return logits.reshape(B, T, -1), _LazyMerged(layer_aux)
+
     def _attention(self, p, h, layer_cache, positions, drop=None):
         cfg = self.cfg
         B, T, d = h.shape
@@ -509,6 +644,9 @@ class MemoryPoolLM:
         if (self.decode and tokens.is_cuda and cache is not None and positions is not None and T == 1 and not train
                 and not pool_off and not route_through_pool and probes is None and not shuffle_pool):
             return self._decode_step_gpu(p, tokens, positions, cache, noise_scale, rngs, input_rows)
+        if (not self.decode and positions is None and not train and not route_through_pool and probes is None
+                and not sparse_grad and self._fused_forward_ok(p, tokens)):
+            return self._forward_gpu(p, tokens, pool_off, noise_scale, shuffle_pool, rngs)
         emb = p["embed"]["embedding"]
         if positions is None:
             x = emb[tokens] + p["pos_embed"][None, :T]

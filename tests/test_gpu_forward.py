@@ -1,0 +1,110 @@
+"""The backbone over whole sequences in plain inference (MemoryPoolLM.apply
+under no_grad): mpl_dense_layers against the oracle's layer_norm, dense,
+gelu_tanh and silu and mpl_causal_attention against softmax attention, both in
+fp64, around the edges of their tiles; and the fused forward against the
+general path, which a call with gradients enabled takes."""
+
+import numpy as np
+import pytest
+import torch
+
+from model_amd import _lib
+from model_amd.model import MemoryPoolLM, ModelConfig, causal_attention, dense_layers
+from oracle import backbone as ob
+
+pytestmark = pytest.mark.gpu
+
+ACTS = {None: lambda v: v, "gelu_tanh": ob.gelu_tanh, "silu": ob.silu}
+
+
+@pytest.mark.parametrize("rows,K,widths,acts,out_in,ln,mul,residual,joined", [
+    (1, 4, [4], [None], False, False, False, False, False),              # the smallest of each
+    (64, 64, [64], [None], False, False, False, True, False),            # one tile, one chunk
+    (65, 68, [68], ["silu"], False, True, False, False, False),          # one past in rows, K and columns
+    (63, 60, [60], ["gelu_tanh"], False, True, True, True, False),       # one short of each
+    (200, 256, [256, 256, 256], [None, None, None], False, True, False, False, True),   # query, key, value
+    (130, 256, [1024, 256], [None, "silu"], False, True, False, False, False),          # router and gate
+    (129, 1024, [256], [None], False, False, False, True, False),        # feed-forward output
+    (100, 300, [20, 4, 132], ["silu", None, "gelu_tanh"], False, True, False, False, False),
+    (70, 128, [516], [None], True, True, False, False, False),           # embedding table layout
+    (70, 36, [100], [None], True, False, True, True, False),
+])
+def test_dense_layers_match_oracle(gpu_lib, rows, K, widths, acts, out_in, ln, mul, residual, joined):
+    """fp32 sums of K terms: within 2e-5 of the result's largest magnitude, as
+    mpl_rows_linear."""
+    rng = np.random.default_rng(rows * 31 + K)
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    x = f32(rows, K) * np.float32(1.5) + np.float32(0.3)
+    Ws = [f32(n, K) * np.float32(K ** -0.5) if out_in else f32(K, n) * np.float32(K ** -0.5) for n in widths]
+    bs = [f32(n) if i % 2 == 0 else None for i, n in enumerate(widths)]
+    lnp = {"scale": 1 + np.float32(0.1) * f32(K), "bias": np.float32(0.1) * f32(K)} if ln else None
+    m = f32(rows, K) if mul else None
+    res = f32(rows, widths[0]) if residual else None
+    cu = lambda t: None if t is None else torch.tensor(t, device="cuda")  # noqa: E731
+    got = dense_layers(cu(x), [(cu(w), cu(b), a) for w, b, a in zip(Ws, bs, acts)], x_mul=cu(m), residual=cu(res),
+                       ln=None if lnp is None else {k: cu(v) for k, v in lnp.items()}, out_in=out_in, joined=joined)
+    a = x.astype(np.float64)
+    if ln:
+        a = ob.layer_norm(a, {k: v.astype(np.float64) for k, v in lnp.items()})
+    if mul:
+        a = a * m.astype(np.float64)
+    want = []
+    for w, b, act, n in zip(Ws, bs, acts, widths):
+        w = w.astype(np.float64)
+        y = ACTS[act](ob.dense(a, {"kernel": w.T if out_in else w, "bias": np.zeros(n) if b is None else b}))
+        want.append(y + res if residual else y)
+    if joined:
+        want = [np.concatenate(want, 1)]
+    for y, g in zip(want, got):
+        np.testing.assert_allclose(g.cpu().numpy(), y, rtol=0, atol=2e-5 * np.abs(y).max())
+
+
+@pytest.mark.parametrize("B,T,H,hd", [(1, 1, 1, 32), (2, 31, 3, 32), (3, 32, 2, 64), (2, 33, 4, 64), (1, 100, 2, 128),
+                                      (2, 129, 1, 64), (1, 300, 2, 32)])
+def test_causal_attention_matches_softmax(gpu_lib, B, T, H, hd):
+    """Scores of hd terms enter an exponential: an absolute error of hd * 2^-24
+    times the largest |q||k| a score, the same relative error a weight; 4e-6
+    covers it for these scores (|s| < 16) with the sums' own."""
+    g = torch.Generator().manual_seed(T + hd)
+    qkv = torch.randn((B, T, 3, H, hd), generator=g)
+    qkv[:, T // 2:, 1] *= 3.0  # sharper rows: the running maximum moves between key blocks
+    got = causal_attention(qkv.reshape(B, T, -1).cuda(), H, hd ** -0.5).cpu().double().reshape(B, T, H, hd)
+    q, k, v = (qkv[:, :, i].double().permute(0, 2, 1, 3) for i in range(3))
+    s = (q * hd ** -0.5) @ k.transpose(-1, -2).contiguous()
+    s = s.masked_fill(~torch.ones((T, T), dtype=torch.bool).tril(), -float("inf"))
+    want = (torch.softmax(s, -1) @ v).permute(0, 2, 1, 3)
+    assert float((got - want).abs().max()) <= 4e-6 * max(1.0, float(s[s > -1e30].abs().max())) * float(v.abs().max())
+
+
+def test_unsupported_shapes_are_reported(gpu_lib):
+    L = _lib.lib()
+    s = torch.cuda.current_stream().cuda_stream
+    assert L.mpl_causal_attention(None, 1, 8, 2, 48, 1.0, None, s) == 4 and b"head_dim" in L.mpl_last_error()
+    with pytest.raises(_lib.MplError, match="width"):
+        dense_layers(torch.zeros((8, 8), device="cuda"), [(torch.zeros((8, 6), device="cuda"), None, None)])
+
+
+@pytest.mark.parametrize("B,T,heads,memory_ffn,use_memory,pool_off", [
+    (3, 40, 2, False, True, False), (1, 1, 4, True, True, False), (2, 65, 4, True, True, True),
+    (2, 33, 2, False, False, False)])
+def test_fused_forward_equals_general_path(gpu_lib, B, T, heads, memory_ffn, use_memory, pool_off):
+    """fp32 tables, so that a change of rounding cannot move a selected slot
+    but at a tie of its scores; the same fp32 rounding through 3 layers, 1e-4
+    as the backbone's test against the oracle."""
+    cfg = ModelConfig(vocab_size=400, max_len=80, d_model=128, n_layers=3, n_heads=heads, ffn_mult=2,
+                      use_memory=use_memory, memory_layers=(0, 2), memory_ffn=memory_ffn, n_sub_keys=24, pool_heads=2,
+                      d_key=32, d_value=64, top_k=8, values_dtype=torch.float32)
+    model = MemoryPoolLM(cfg)
+    params = model.init(3)
+    tokens = torch.randint(0, 400, (B, T), generator=torch.Generator().manual_seed(1)).cuda()
+    with torch.no_grad():
+        assert model._fused_forward_ok(params["params"], tokens)
+        got, aux = model.apply(params, tokens, pool_off=pool_off)
+    want, aux2 = model.apply(params, tokens, pool_off=pool_off)  # gradients enabled: the general path
+    assert not model._fused_forward_ok(params["params"], tokens)
+    torch.testing.assert_close(got, want.detach(), rtol=1e-4, atol=1e-4)
+    if use_memory and not pool_off:
+        assert all(torch.equal(a, b) for a, b in zip(aux["slots"], aux2["slots"]))
+    # transforms and modes take the general path
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        assert not model._fused_forward_ok(params["params"], tokens)
