@@ -38,6 +38,9 @@ NORM_EPS = 1e-6
 # The routed query gradient inside the dense balance pass where it applies
 # (mpl_lookup_bwd_dense_queries); False keeps the separate query pass.
 FUSED_QUERY_BWD = True
+# Bytes of a lookup's workspace up to which it shares the allocation of the
+# selection lists, which a backward keeps.
+_WS_WITH_LISTS = 1 << 20
 # In that pass, fp16 operand packs made from the raw queries (normalised in
 # the pack, the same bits as the fp32 q_hat pass); False packs q_hat.
 RAW_QUERY_PACK = True
@@ -52,7 +55,7 @@ def _dtype_code(dt: torch.dtype) -> int:
 
 
 def _capturing() -> bool:
-    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
 
 class _KeyCache:
@@ -75,7 +78,7 @@ class _KeyCache:
 
     def get(self, sub_keys: torch.Tensor, score_code: int):
         key = (sub_keys.data_ptr(), sub_keys._version, tuple(sub_keys.shape), score_code)
-        if _capturing() and not self.frozen:
+        if not self.frozen and _capturing():
             return self._pack(sub_keys, score_code)
         if key != self.key or sub_keys is not self.src:
             self.k_hat, self.packed = self._pack(sub_keys, score_code)
@@ -138,20 +141,42 @@ class LazyAux(dict):
         return self
 
 
-class _Result(dict):
-    """The lookup's result; "q_hat" (fp32 normalised queries, which the
-    scoring kernel does not need) is computed on first access."""
+class _Views(dict):
+    """What only the statistics and a backward read of a lookup, each made on
+    first access: the views "q" [M, H, 2, half], "slots" and "weights"
+    [M, H, k], "sub_idx" and "sub_scores" [M, H, 2, k] and "flat_idx"
+    [M, H, k] (the last three parts of one allocation), and "q_hat", the fp32
+    normalised queries, which the scoring kernel does not need.  A decode loop
+    then does not pay a microsecond of host time for each."""
+
+    def __init__(self, make: Dict[str, Any]):
+        super().__init__()
+        self._make = make
 
     def __missing__(self, key):
-        if key != "q_hat":
-            raise KeyError(key)
+        v = self[key] = self._q_hat() if key == "q_hat" else self._make[key]()
+        return v
+
+    def _q_hat(self):
         q = self["q"]
         M, H, _, half = q.shape
         q_hat = torch.empty_like(q)
         check(_lib.lib().mpl_l2_normalize(ptr(q), M * H * 2, half, NORM_EPS, ptr(q_hat), None, None,
                                           _lib.stream_ptr(q.device)), "mpl_l2_normalize")
-        self["q_hat"] = q_hat
         return q_hat
+
+
+class _Result(dict):
+    """The lookup's result; keys it does not hold are its _Views (shared with
+    the aux, which refers to them and not to this dict: no reference cycle
+    keeps a call's tensors until a garbage collection)."""
+
+    def __init__(self, eager: Dict[str, Any], views: _Views):
+        super().__init__(eager)
+        self._views = views
+
+    def __missing__(self, key):
+        return self._views[key]
 
 
 def routing_seed(rngs: Optional[Dict[str, Any]]) -> int:
@@ -261,7 +286,7 @@ class MemoryPool:
         computed on the device (no host read), cached per parameter version
         outside graph capture."""
         key = (log_temperature.data_ptr(), log_temperature._version)
-        if ((_capturing() and not self._keys.frozen) or key != self._temp_key
+        if ((not self._keys.frozen and _capturing()) or key != self._temp_key
                 or log_temperature is not self._temp_src):
             lt = log_temperature.detach().reshape(1).to(torch.float32).contiguous()
             t = torch.empty(1, dtype=torch.float32, device=lt.device)
@@ -352,16 +377,19 @@ class MemoryPool:
         the noise draw and the noisy selection."""
         H, n, k, d = self.heads, self.n_sub_keys, self.top_k, self.d_value
         half = self.d_key // 2
-        lead = tuple(queries.shape[:-2])
-        if tuple(queries.shape[-2:]) != (H, self.d_key):
-            raise ValueError(f"queries must be [..., {H}, {self.d_key}], got {tuple(queries.shape)}")
+        shape = tuple(queries.shape)
+        lead = shape[:-2]
+        if shape[-2:] != (H, self.d_key):
+            raise ValueError(f"queries must be [..., {H}, {self.d_key}], got {shape}")
         dev = queries.device
         if dev.type != "cuda":
             raise RuntimeError("MemoryPool runs on the GPU only (libmpl.so); got a tensor on " + str(dev))
         L = _lib.lib()
         stream = _lib.stream_ptr(dev)
-        q = queries.detach().reshape(-1, H, 2, half).float().contiguous()
-        M = q.shape[0]
+        q = queries.detach()
+        if q.dtype != torch.float32 or not q.is_contiguous():
+            q = q.reshape(-1, H, 2, half).float().contiguous()
+        M = q.numel() // (H * self.d_key)
         score_code = _dtype_code(self.score_dtype)
         # the scoring kernel normalises the raw queries itself (and computes
         # q_len with query_scale); the fp32 q_hat is produced only on demand
@@ -387,13 +415,22 @@ class MemoryPool:
             gumbel = gumbel.reshape(M, H, 2, n).float().contiguous()
 
         ws_bytes = L.mpl_score_select_workspace_bytes(M, H, n, half, k)
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        sub_idx = torch.empty((M, H, 2, k), dtype=torch.int32, device=dev)
-        sub_scores = torch.empty((M, H, 2, k), dtype=torch.float32, device=dev)
-        flat_idx = torch.empty((M, H, k), dtype=torch.int32, device=dev)
-        slots = torch.empty((M, H, k), dtype=torch.int32, device=dev)
-        weights = torch.empty((M, H, k), dtype=torch.float32, device=dev)
-        out = torch.empty((M, d), dtype=torch.float32, device=dev)
+        # sub_idx, sub_scores and flat_idx as parts of one buffer, each from a
+        # multiple of 64 words; a small workspace lies behind them, a large
+        # one is given back when the call returns
+        mhk = M * H * k
+        part = (2 * mhk + 63) // 64 * 64
+        words = 2 * part + (mhk + 63) // 64 * 64
+        ws = None
+        if ws_bytes > _WS_WITH_LISTS:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        lists = torch.empty(words if ws is not None else words + (ws_bytes + 3) // 4, dtype=torch.int32, device=dev)
+        sub_idx = lists.data_ptr()
+        ws_at = ws.data_ptr() if ws is not None else sub_idx + 4 * words
+        sub_scores, flat_idx = sub_idx + 4 * part, sub_idx + 8 * part
+        slots = torch.empty((*lead, H, k), dtype=torch.int32, device=dev)
+        weights = torch.empty((*lead, H, k), dtype=torch.float32, device=dev)
+        out = torch.empty((*lead, d), dtype=torch.float32, device=dev)
         staged = None
         if not self.host_pool:
             # selection and value read in one call (memory.py:132-193): with
@@ -403,48 +440,55 @@ class MemoryPool:
                 raise TypeError("values must be a contiguous float16/float32 [n*n, d_value] tensor")
             if tuple(values.shape) != (self.pool_size, d):
                 raise ValueError(f"values must be [{self.pool_size}, {d}], got {tuple(values.shape)}")
-            check(L.mpl_lookup(ptr(q), q_mode, ptr(q_len), ptr(packed), M, H, n, half, k, score_code,
-                               ptr(T), ptr(gumbel), ptr(noise_coef), ptr(ws), ws_bytes, ptr(sub_idx),
-                               ptr(sub_scores), ptr(flat_idx), ptr(slots), ptr(weights),
-                               ptr(values), _dtype_code(values.dtype), d, int(bool(shuffle_reads)), ptr(out),
+            check(L.mpl_lookup(q.data_ptr(), q_mode, ptr(q_len), packed.data_ptr(), M, H, n, half, k, score_code,
+                               T.data_ptr(), ptr(gumbel), ptr(noise_coef), ws_at, ws_bytes, sub_idx,
+                               sub_scores, flat_idx, slots.data_ptr(), weights.data_ptr(),
+                               values.data_ptr(), _dtype_code(values.dtype), d, int(bool(shuffle_reads)),
+                               out.data_ptr(),
                                stream), "mpl_lookup")
         else:
             check(L.mpl_score_select(ptr(q), q_mode, ptr(q_len), ptr(packed), M, H, n, half, k, score_code,
-                                     ptr(T), ptr(gumbel), ptr(noise_coef), ptr(ws), ws_bytes, ptr(sub_idx),
-                                     ptr(sub_scores), ptr(flat_idx), ptr(slots), ptr(weights), stream),
+                                     ptr(T), ptr(gumbel), ptr(noise_coef), ws_at, ws_bytes, sub_idx,
+                                     sub_scores, flat_idx, ptr(slots), ptr(weights), stream),
                   "mpl_score_select")
             # memory.py:182-183 (hp.fetch): the unique rows cross the host
             # link once into device memory; the weighted sum reads them there
             from . import host_pool as hp
-            read = slots
+            read = slots.reshape(M, H, k)
             if shuffle_reads:  # memory.py:179
                 N = self.pool_size
-                read = ((slots.long() + N // 2 + 1) % N).to(torch.int32)
+                read = ((read.long() + N // 2 + 1) % N).to(torch.int32)
             rows, inverse, _ = hp.get(self.host_pool).stage(read)
             staged = (rows, inverse.reshape(M, H, k))
             check(L.mpl_gather_wsum(ptr(rows), _dtype_code(rows.dtype), max(rows.shape[0], 1), d, ptr(staged[1]),
                                     ptr(weights), M, H * k, 0, ptr(out), stream), "mpl_gather_wsum")
 
         noisy = gumbel is not None
-        res = _Result()
+
+        views = _Views({
+            "q": lambda: q.reshape(M, H, 2, half),
+            "slots": lambda: slots.reshape(M, H, k),
+            "weights": lambda: weights.reshape(M, H, k),
+            "sub_idx": lambda: lists[:2 * mhk].view(M, H, 2, k),
+            "sub_scores": lambda: lists[part:part + 2 * mhk].view(torch.float32).view(M, H, 2, k),
+            "flat_idx": lambda: lists[2 * part:2 * part + mhk].view(M, H, k),
+        })
 
         def stats():
-            return self._routing_stats(params, res, k_hat, T, q_len, sub_idx, slots, weights,
-                                       noisy, packed, score_code, M, early)
+            return self._routing_stats(params, views, k_hat, T, q_len, views["sub_idx"], slots, weights, noisy,
+                                       packed, score_code, M, early)
 
         aux = LazyAux({
-            "slots": slots.reshape(*lead, H, k),
-            "weights": weights.reshape(*lead, H, k),
+            "slots": slots,
+            "weights": weights,
             "temperature": T.reshape(()),
-        }, stats, queries=lambda: res["q_hat"], top1_weight=lambda: weights.max(-1).values.mean(),
+        }, stats, queries=lambda: views["q_hat"], top1_weight=lambda: weights.max(-1).values.mean(),
             slot_counts=lambda: self._slot_counts(slots, M))
-        res.update({
-            "out": out.reshape(*lead, d), "aux": aux, "q": q, "q_len": q_len,
-            "k_hat": k_hat, "packed": packed, "score_code": score_code, "temperature": T, "sub_idx": sub_idx, "sub_scores": sub_scores,
-            "flat_idx": flat_idx, "slots": slots, "weights": weights, "gumbel": gumbel, "staged": staged,
-            "noise_coef": noise_coef,
-        })
-        return res
+        return _Result({
+            "out": out, "aux": aux, "q_len": q_len,
+            "k_hat": k_hat, "packed": packed, "score_code": score_code, "temperature": T, "gumbel": gumbel,
+            "staged": staged, "noise_coef": noise_coef,
+        }, views)
 
     # ------------------------------------------------------------- stats
     def _routing_stats(self, params, res, k_hat, T, q_len, sub_idx, slots, weights, noisy,
