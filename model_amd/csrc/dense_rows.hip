@@ -7,24 +7,28 @@
 //
 // W_i is [K, N_i] (a Dense kernel) or [N_i, K] (the embedding table).  A
 // workgroup of 4 waves owns a 64 x 64 tile of one layer's output, each wave a
-// 32 x 32 block on v_mfma_f32_32x32x2_f32.  K runs in chunks of 32 through
-// LDS: the next chunk's 16-byte loads are in flight while this one's MFMAs
-// run.  The contraction is permuted so that one 16-byte LDS read of a row
-// feeds four MFMAs (lanes of half h take dims 4h .. 4h+3 of each 8), for x
-// and for [N, K] weights; [K, N] weights are read as they lie, one dword a
-// MFMA.  LayerNorm statistics (mean, then the centred variance) are wave sums
-// over the tile's own rows before the first chunk.  One order of the sums for
-// every tile, so results do not depend on which layers share a launch.
+// 32 x 32 block on v_mfma_f32_32x32x2_f32.  K runs in chunks of 32 through two
+// LDS buffers: while a chunk's MFMAs run, the next one goes into the other
+// buffer and the 16-byte loads of the one three later are sent (two register
+// sets in flight), and the last four MFMAs cover the next chunk's LDS reads;
+// one barrier a chunk.  The contraction is permuted so that one 16-byte LDS
+// read of a row feeds four MFMAs (lanes of half h take dims 4h .. 4h+3 of each
+// 8), for x and for [N, K] weights; [K, N] weights are read as they lie, one
+// dword a MFMA.  LayerNorm statistics (mean, then the centred variance) are
+// wave sums over the tile's own rows before the first chunk.  One order of the
+// sums for every tile, so results do not depend on which layers share a launch.
 //
-// Bound: the fp32 MFMAs (64 cycles each, 16 a wave and chunk) at two thirds of
-// their rate; what it saves are the passes around a product.  Measured, 4,096
-// rows, us (the library's product alone): K = 256, N = 768 with LayerNorm 31.1
-// (23.5), N = 256 11.5 (9.6), K = 1,024, N = 256 31.0 (21.7); a separate
-// LayerNorm takes 8, each elementwise pass 4 to 10, and the whole backbone
-// over 16 x 256 tokens goes from 1,490 to 935 with causal_attn.hip.  Chunks of
-// 64 columns, two register sets of chunks in flight, 16x16x4 MFMAs and two
-// groups of waves splitting K measured no faster.
+// Bound: the fp32 MFMAs (64 cycles each, 16 a wave and chunk: 0.43 us), with
+// 6 us of launch, first loads and epilogue around them and 5 us for LayerNorm.
+// A chunk takes 0.56 us at one wave a SIMD; 0.47 without the staging between
+// the MFMAs.  Measured, 4,096 rows, us, with one LDS buffer and one register
+// set -> now: K = 256, N = 768 with LayerNorm 30.5 -> 27.5, N = 1,024 with
+// LayerNorm and GELU 41.7 -> 36.8, N = 256 13.2 -> 11.5, K = 1,024, N = 256
+// 34.2 -> 25.9.  Chunks of 64 columns, 16x16x4 MFMAs and two groups of waves
+// splitting K measured no faster.
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "topk.h"
@@ -53,6 +57,7 @@ struct DenseArgs {
   const float* residual;  // one layer only, its output's shape
   int64_t rows;
   int K, count;
+  uint32_t tiles;  // column tiles of all the layers
   float eps;
   DenseLayer layer[kMaxLayers];
 };
@@ -98,17 +103,23 @@ __device__ __forceinline__ float4 keep_if(float4 v, bool ok) {
 }
 
 template <int LAYOUT, bool LN, bool MUL>
-__global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs p) {
-  __shared__ float sa[kTM * kPA];
-  __shared__ float sw[LAYOUT == MPL_W_IN_OUT ? kKC * kPW : kTN * kPA];
+__global__ __launch_bounds__(256, MUL ? 3 : 4) void dense_rows_kernel(DenseArgs p) {
+  constexpr int SA = kTM * kPA, SW = LAYOUT == MPL_W_IN_OUT ? kKC * kPW : kTN * kPA;
+  __shared__ float sa[2 * SA];
+  __shared__ float sw[2 * SW];
   __shared__ float smean[kTM], srstd[kTM];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t m0 = (int64_t)blockIdx.y * kTM;
+  // Workgroups go to the 8 XCDs in turn; each XCD takes a run of neighbouring
+  // row tiles with all their column tiles, so its L2 holds an eighth of x.
+  const uint32_t id = blockIdx.x, full = gridDim.x / 8 * 8;
+  const uint32_t at = id < full ? (id & 7) * (full / 8) + (id >> 3) : id;
+  const int64_t m0 = (int64_t)(at / p.tiles) * kTM;
+  const int tile = (int)(at % p.tiles);
   int li = 0;
-  if (p.count > 1 && (int)blockIdx.x >= p.layer[1].tile0) li = 1;
-  if (p.count > 2 && (int)blockIdx.x >= p.layer[2].tile0) li = 2;
+  if (p.count > 1 && tile >= p.layer[1].tile0) li = 1;
+  if (p.count > 2 && tile >= p.layer[2].tile0) li = 2;
   const DenseLayer L = p.layer[li];
-  const int n0 = ((int)blockIdx.x - L.tile0) * kTN;
+  const int n0 = (tile - L.tile0) * kTN;
   const int K = p.K;
 
   // Thread's 16-byte pieces of a chunk: of x, rows tid/16 + 16 i, columns
@@ -118,32 +129,62 @@ __global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs p) {
   constexpr int NW = LAYOUT == MPL_W_IN_OUT ? kKC / 16 : NA;
   const int pr = tid / CA, pc = 4 * (tid % CA);
   const int wr = LAYOUT == MPL_W_IN_OUT ? tid >> 4 : pr, wc = LAYOUT == MPL_W_IN_OUT ? 4 * (tid & 15) : pc;
-  float4 ra[NA], rw[NW], rm[MUL ? NA : 1];
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
-    const int kc = min(k0 + pc, K - 4);
+  // These point at the thread's pieces of chunk `at_k` (which the main loop
+  // advances); a chunk that may reach past K is read clamped.
+  const float *xp[NA], *mp[MUL ? NA : 1], *wp[NW];
+  int at_k = 0;
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int64_t row = min(m0 + pr + RA * i, p.rows - 1) * K;
+    xp[i] = p.x + row + pc;
+    if (MUL) mp[MUL ? i : 0] = p.x_mul + row + pc;
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i)
+    wp[i] = LAYOUT == MPL_W_IN_OUT ? L.w + min(n0 + wc, L.N - 4) + (int64_t)(wr + 16 * i) * L.N
+                                   : L.w + (int64_t)min(n0 + wr + RA * i, L.N - 1) * K + pc;
+  // Whole: the main loop's addresses step along and nothing is masked (10 %
+  // of a K = 1,024 layer).  Not with LayerNorm, whose registers would spill
+  // (29.4 us against 27.5 at N = 768).
+  using Yes = std::true_type;
+  using No = std::false_type;
+  using Whole = std::integral_constant<bool, !LN>;
+  struct Pieces {
+    float4 a[NA], w[NW], m[MUL ? NA : 1];
+  };
+  Pieces set0, set1;  // of two chunks, in flight
+  float4 rg, rb;
+  auto fetch = [&](Pieces& r, int k0, auto WHOLE) __attribute__((always_inline)) {
+    const int kd = k0 - at_k;
+    const int kc = WHOLE ? kd : min(k0 + pc, K - 4) - pc - at_k;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      const int64_t row = min(m0 + pr + RA * i, p.rows - 1);
-      ra[i] = *(const float4*)(p.x + row * K + kc);
-      if (MUL) rm[MUL ? i : 0] = *(const float4*)(p.x_mul + row * K + kc);
+      r.a[i] = *(const float4*)(xp[i] + kc);
+      if (MUL) r.m[MUL ? i : 0] = *(const float4*)(mp[MUL ? i : 0] + kc);
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       if (LAYOUT == MPL_W_IN_OUT)
-        rw[i] = *(const float4*)(L.w + (int64_t)min(k0 + wr + 16 * i, K - 1) * L.N + min(n0 + wc, L.N - 4));
+        r.w[i] = *(const float4*)(wp[i] + (int64_t)((WHOLE ? k0 : min(k0, K - 1 - wr - 16 * i)) - at_k) * L.N);
       else
-        rw[i] = *(const float4*)(L.w + (int64_t)min(n0 + wr + RA * i, L.N - 1) * K + kc);
+        r.w[i] = *(const float4*)(wp[i] + kc);
     }
   };
-  fetch(0);
+  auto fetch_ln = [&](int k0) __attribute__((always_inline)) {
+    const int kc = min(k0 + pc, K - 4);
+    rg = *(const float4*)(p.ln_scale + kc);
+    rb = *(const float4*)(p.ln_bias + kc);
+  };
+  if (!LN) fetch(set0, 0, No{});
 
   if (LN) {
     // 16 rows a wave, all requested at once: one memory round trip for up to
     // 256 columns, which then stay in registers for the second pass
     const float inv = 1.f / (float)K;
     const float* src[16];
+    const int w0 = 16 * __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) src[i] = p.x + min(m0 + 16 * wave + i, p.rows - 1) * K;
+    for (int i = 0; i < 16; ++i) src[i] = p.x + min(m0 + w0 + i, p.rows - 1) * K;
     float4 t[16];
     float s[16], v[16];
     auto rows16 = [&](int c0) __attribute__((always_inline)) {
@@ -188,34 +229,37 @@ __global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs p) {
     __syncthreads();
   }
 
-  auto stage = [&](int k0) __attribute__((always_inline)) {
+  if (LN) {  // the statistics take the registers until here
+    fetch(set0, 0, No{});
+    fetch_ln(0);
+  }
+  fetch(set1, kKC, No{});  // past K: clamped, and not used
+  float mu[NA], rs[NA];
+#pragma unroll
+  for (int i = 0; LN && i < NA; ++i) {
+    mu[i] = smean[pr + RA * i];
+    rs[i] = srstd[pr + RA * i];
+  }
+  auto stage = [&](const Pieces& r, int k0, int buf, auto WHOLE) __attribute__((always_inline)) {
     const bool kok = k0 + pc < K;
-    const int kc = min(k0 + pc, K - 4);
-    float4 g = make_float4(0.f, 0.f, 0.f, 0.f), be = g;
-    if (LN) {
-      g = *(const float4*)(p.ln_scale + kc);
-      be = *(const float4*)(p.ln_bias + kc);
-    }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      float4 a = ra[i];
-      if (LN) {
-        const float mu = smean[pr + RA * i], rs = srstd[pr + RA * i];
-        a = make_float4((a.x - mu) * rs * g.x + be.x, (a.y - mu) * rs * g.y + be.y, (a.z - mu) * rs * g.z + be.z,
-                        (a.w - mu) * rs * g.w + be.w);
-      }
+      float4 a = r.a[i];
+      if (LN)
+        a = make_float4((a.x - mu[i]) * rs[i] * rg.x + rb.x, (a.y - mu[i]) * rs[i] * rg.y + rb.y,
+                        (a.z - mu[i]) * rs[i] * rg.z + rb.z, (a.w - mu[i]) * rs[i] * rg.w + rb.w);
       if (MUL) {
-        const float4 q = rm[MUL ? i : 0];
+        const float4 q = r.m[MUL ? i : 0];
         a = make_float4(a.x * q.x, a.y * q.y, a.z * q.z, a.w * q.w);
       }
-      *(float4*)(sa + (pr + RA * i) * kPA + pc) = keep_if(a, kok);
+      *(float4*)(sa + buf * SA + (pr + RA * i) * kPA + pc) = WHOLE ? a : keep_if(a, kok);
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       if (LAYOUT == MPL_W_IN_OUT)
-        *(float4*)(sw + (wr + 16 * i) * kPW + wc) = keep_if(rw[i], k0 + wr + 16 * i < K);
+        *(float4*)(sw + buf * SW + (wr + 16 * i) * kPW + wc) = WHOLE ? r.w[i] : keep_if(r.w[i], k0 + wr + 16 * i < K);
       else
-        *(float4*)(sw + (wr + RA * i) * kPA + wc) = keep_if(rw[i], kok);
+        *(float4*)(sw + buf * SW + (wr + RA * i) * kPA + wc) = WHOLE ? r.w[i] : keep_if(r.w[i], kok);
     }
   };
 
@@ -224,29 +268,77 @@ __global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs p) {
   const float* pa = sa + (32 * wm + col) * kPA + 4 * h;
   const float* pw = LAYOUT == MPL_W_IN_OUT ? sw + 4 * h * kPW + 32 * wn + col : sw + (32 * wn + col) * kPA + 4 * h;
   f32x16 acc = f32x16{};
-  for (int k0 = 0; k0 < K; k0 += kKC) {
-    if (k0 > 0) __syncthreads();  // every wave has read the chunk before
-    stage(k0);
-    __syncthreads();
-    if (k0 + kKC < K) fetch(k0 + kKC);
-    float4 a[kKC / 8], b[kKC / 8];  // the chunk's operands, requested before the first MFMA
+  constexpr int G = kKC / 8;  // groups of four MFMAs a chunk
+  float4 oa[G], ob[G];        // the chunk's operands
+  auto operands = [&](int g, int buf) __attribute__((always_inline)) {
+    const float *ca = pa + buf * SA + 8 * g, *cw = pw + buf * SW;
+    oa[g] = *(const float4*)ca;
+    if (LAYOUT == MPL_W_IN_OUT)
+      ob[g] = make_float4(cw[(8 * g + 0) * kPW], cw[(8 * g + 1) * kPW], cw[(8 * g + 2) * kPW], cw[(8 * g + 3) * kPW]);
+    else
+      ob[g] = *(const float4*)(cw + 8 * g);
+  };
+  auto mfma4 = [&](float4 a, float4 b) __attribute__((always_inline)) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+  };
+  // One chunk, its operands in registers: the MFMAs of all groups but the
+  // last with the next chunk's way into the other buffer between them (r, and
+  // with FETCH the loads of the chunk two later into r); then the next
+  // chunk's operands are on their way while the last group runs.
+  auto chunk = [&](Pieces& r, int k0, int buf, auto FETCH, auto WHOLE) __attribute__((always_inline)) {
+    stage(r, k0 + kKC, buf ^ 1, WHOLE);
+    if (FETCH) fetch(r, k0 + 3 * kKC, WHOLE);
+    if (LN) fetch_ln(k0 + 2 * kKC);
 #pragma unroll
-    for (int g = 0; g < kKC / 8; ++g) {
-      a[g] = *(const float4*)(pa + 8 * g);
-      if (LAYOUT == MPL_W_IN_OUT)
-        b[g] = make_float4(pw[(8 * g + 0) * kPW], pw[(8 * g + 1) * kPW], pw[(8 * g + 2) * kPW], pw[(8 * g + 3) * kPW]);
-      else
-        b[g] = *(const float4*)(pw + 8 * g);
+    for (int g = 0; g < G - 1; ++g) mfma4(oa[g], ob[g]);
+    // MFMAs wait for one another, and what follows one in program order
+    // waits with it: a few of the other instructions after each
+#pragma unroll
+    for (int g = 0; g < 4 * (G - 1); ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x002, LN ? 8 : 5, 0);           // VALU
+      if (g & 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);         // LDS write
+      if (g & 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);         // load
     }
+    __syncthreads();
+    const float4 la = oa[G - 1], lb = ob[G - 1];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int g = 0; g < kKC / 8; ++g) {
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].x, b[g].x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].y, b[g].y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].z, b[g].z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[g].w, b[g].w, acc, 0, 0, 0);
+    for (int g = 0; g < G; ++g) operands(g, buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma4(la, lb);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  stage(set0, 0, 0, No{});
+  fetch(set0, 2 * kKC, No{});
+  if (LN) fetch_ln(kKC);
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < G; ++g) operands(g, 0);
+  int k0 = 0;
+  for (; k0 + 5 * kKC <= K; k0 += 2 * kKC) {  // what is fetched here lies below K
+    chunk(set1, k0, 0, Yes{}, Whole{});
+    chunk(set0, k0 + kKC, 1, Yes{}, Whole{});
+    if (LN) continue;
+    at_k += 2 * kKC;
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      xp[i] += 2 * kKC;
+      if (MUL) mp[MUL ? i : 0] += 2 * kKC;
     }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) wp[i] += LAYOUT == MPL_W_IN_OUT ? (int64_t)2 * kKC * L.N : (int64_t)2 * kKC;
   }
+  // up to five chunks left
+  if (k0 + kKC < K) chunk(set1, k0, 0, Yes{}, No{});
+  if (k0 + 2 * kKC < K) chunk(set0, k0 + kKC, 1, Yes{}, No{});
+  if (k0 + 3 * kKC < K) chunk(set1, k0 + 2 * kKC, 0, No{}, No{});
+  if (k0 + 4 * kKC < K) chunk(set0, k0 + 3 * kKC, 1, No{}, No{});
+#pragma unroll
+  for (int g = 0; g < G; ++g) mfma4(oa[g], ob[g]);
 
   const int n = n0 + 32 * wn + col;
   if (n >= L.N) return;
@@ -299,7 +391,7 @@ extern "C" int mpl_dense_layers(const float* x, const float* x_mul, const float*
   MPL_REQUIRE(aligned16(x) && aligned16(x_mul) && aligned16(ln_scale) && aligned16(ln_bias), MPL_EINVAL,
               "mpl_dense_layers: x, x_mul, ln_scale and ln_bias must be 16-byte aligned");
   MPL_REQUIRE(residual == nullptr || count == 1, MPL_EINVAL, "mpl_dense_layers: a residual goes with one layer");
-  DenseArgs a{x, x_mul, ln_scale, ln_bias, residual, rows, K, count, ln_eps, {}};
+  DenseArgs a{x, x_mul, ln_scale, ln_bias, residual, rows, K, count, 0, ln_eps, {}};
   int64_t tiles = 0;
   for (int i = 0; i < count; ++i) {
     DenseLayer& L = a.layer[i];
@@ -320,7 +412,10 @@ extern "C" int mpl_dense_layers(const float* x, const float* x_mul, const float*
     tiles += cdiv(L.N, kTN);
   }
   MPL_REQUIRE(tiles < ((int64_t)1 << 31), MPL_EUNSUPPORTED, "mpl_dense_layers: too many columns");
-  const dim3 grid((unsigned)tiles, (unsigned)cdiv(rows, kTM));
+  a.tiles = (uint32_t)tiles;
+  const int64_t groups = tiles * cdiv(rows, kTM);
+  MPL_REQUIRE(groups < ((int64_t)1 << 31), MPL_EUNSUPPORTED, "mpl_dense_layers: too many tiles");
+  const dim3 grid((unsigned)groups);
   if (weight_layout == MPL_W_OUT_IN) launch_dense<MPL_W_OUT_IN>(a, grid, (hipStream_t)stream);
   else launch_dense<MPL_W_IN_OUT>(a, grid, (hipStream_t)stream);
   return check_launch("mpl_dense_layers");

@@ -59,6 +59,29 @@ def test_dense_layers_match_oracle(gpu_lib, rows, K, widths, acts, out_in, ln, m
         np.testing.assert_allclose(g.cpu().numpy(), y, rtol=0, atol=2e-5 * np.abs(y).max())
 
 
+@pytest.mark.parametrize("out_in,ln,mul", [(False, False, False), (True, False, False), (False, True, False),
+                                           (False, False, True), (True, True, True)])
+def test_dense_layers_every_chunk_count(gpu_lib, out_in, ln, mul):
+    """The contraction runs in chunks of 32, a main loop of two at a time and
+    up to five after it: every count from one chunk to eleven, whole and with
+    a rest, on more row tiles than the 8 XCDs and a rest."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    R = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    rows, N = 64 * 9 + 5, 68
+    for K in sorted({k for c in range(1, 12) for k in (32 * c - 28, 32 * c)}):
+        x, w, b = R(rows, K), R(N, K) if out_in else R(K, N), R(N)
+        m = R(rows, K) if mul else None
+        lnp = {"scale": R(K), "bias": R(K)} if ln else None
+        got, = dense_layers(x, [(w, b, None)], ln=lnp, x_mul=m, out_in=out_in)
+        a = x.double()
+        if ln:
+            a = torch.nn.functional.layer_norm(a, (K,), lnp["scale"].double(), lnp["bias"].double(), 1e-6)
+        a = a * m.double() if mul else a
+        want = a @ (w.double().t() if out_in else w.double()) + b.double()
+        # fp32 sums of K terms, as above
+        assert float((got - want).abs().max()) <= 2e-5 * float(want.abs().max()), K
+
+
 @pytest.mark.parametrize("B,T,H,hd", [(1, 1, 1, 32), (2, 31, 3, 32), (3, 32, 2, 64), (2, 33, 4, 64), (1, 100, 2, 128),
                                       (2, 129, 1, 64), (1, 300, 2, 32)])
 def test_causal_attention_matches_softmax(gpu_lib, B, T, H, hd):
