@@ -268,6 +268,23 @@ int mpl_gather_rows(const void* table, int dtype, int64_t N, int d, const int32_
 int mpl_host_device_pointer(void* host_ptr, void** dev_ptr);
 
 /*
+ * out[idx[i], :] = rows[i, :] for i < min(count, *count_dev) (count_dev may be
+ * NULL) and idx[i] in [0, N); other entries are skipped and the rest of out is
+ * left as it is.  rows [count, d], out [N, d] fp32, idx without repeats: the
+ * merged rows of mpl_merge_rows as a dense gradient of the table.
+ */
+int mpl_scatter_rows(const float* rows, const int32_t* idx, int64_t count, const int32_t* count_dev, int d, int64_t N,
+                     float* out, void* stream);
+
+/*
+ * Copies `count` (at most 12) arrays of 32-bit words in one launch: words[i]
+ * words from srcs[i] to dsts[i].  srcs, dsts (tables of device pointers) and
+ * words (int64_t) are read on the host before the call returns.  The arrays
+ * must not overlap.
+ */
+int mpl_copy_arrays(const void* srcs, const void* dsts, const void* words, int count, void* stream);
+
+/*
  * train.py:146-172 (fetched_row_grads + _merge_rows): gradient rows of the
  * fetched pool rows.  Fetch p in [0, P) of token p / fetches_per_token reads
  * slot slots[p] with weight weights[p] (weights == NULL: 1).  With

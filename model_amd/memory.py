@@ -856,14 +856,15 @@ def _lookup_backward(pool, res, internal, sub_keys, values, shapes, g_out, g_bal
     dv = None
     if need_dv:
         N = pool.pool_size
-        sl = res["slots"].long()
+        sl = res["slots"]
         if shuffle_reads:
-            sl = (sl + N // 2 + 1) % N
+            sl = ((sl.long() + N // 2 + 1) % N).to(torch.int32)
         from .rows import merge_fetches
-        m = merge_fetches(sl.to(torch.int32), res["weights"], g_out, N)
-        dv_ext = torch.zeros((N + 1, d), dtype=torch.float32, device=dev)
-        dv_ext.index_copy_(0, m.uniq.long(), m.rows)  # padding rows (all zero) land on row N
-        dv = dv_ext[:N].to(values.dtype)
+        m = merge_fetches(sl, res["weights"], g_out, N, zero_padding=False)
+        dv = torch.zeros((N, d), dtype=torch.float32, device=dev)
+        check(L.mpl_scatter_rows(ptr(m.rows), ptr(m.uniq), m.uniq.numel(), ptr(m.num_unique), d, N, ptr(dv), stream),
+              "mpl_scatter_rows")
+        dv = dv.to(values.dtype)
 
     return dq.reshape(q_shape).to(q_dtype), dk.to(k_dtype), dlt.reshape(()).to(t_dtype), dv
 

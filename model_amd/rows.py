@@ -105,6 +105,34 @@ def merge_rows(slots: torch.Tensor, contribs: torch.Tensor, pool_size: int):
     return m.uniq, m.rows
 
 
+def _stacked(*groups):
+    """torch.cat of each group of tensors (along their first dimension), all
+    in one launch (mpl_copy_arrays: 7 us for two layers of 4,096 tokens, where
+    the three concatenations take 20) where they are contiguous 32-bit arrays
+    of one dtype and trailing shape a group on one GPU."""
+    dev = groups[0][0].device
+    plain = dev.type == "cuda" and sum(len(g) for g in groups) <= 12 and all(
+        type(t) is torch.Tensor and t.dtype == g[0].dtype and t.dtype in (torch.int32, torch.float32)
+        and t.device == dev and t.is_contiguous() and not t.is_neg() and t.shape[1:] == g[0].shape[1:] for g in groups for t in g)
+    if not plain:
+        return [torch.cat(g) for g in groups]
+    outs, src, dst, words = [], [], [], []
+    for g in groups:
+        out = torch.empty((sum(t.shape[0] for t in g), *g[0].shape[1:]), dtype=g[0].dtype, device=dev)
+        at = out.data_ptr()
+        for t in g:
+            src.append(t.data_ptr())
+            dst.append(at)
+            words.append(t.numel())
+            at += 4 * t.numel()
+        outs.append(out)
+    n = len(src)
+    table = lambda kind, v: C.cast((kind * n)(*v), C.c_void_p)  # noqa: E731
+    check(_lib.lib().mpl_copy_arrays(table(C.c_void_p, src), table(C.c_void_p, dst), table(C.c_int64, words), n,
+                                     _lib.stream_ptr(dev)), "mpl_copy_arrays")
+    return outs
+
+
 def fetched_row_grads_full(aux: Dict, probe_grads, layers: Sequence[int], pool_size: int,
                            zero_padding: bool = True, slot_counts: Optional[torch.Tensor] = None) -> MergedRows:
     """train.py:146-163 with the extra outputs (row norms, distinct count,
@@ -119,8 +147,7 @@ def fetched_row_grads_full(aux: Dict, probe_grads, layers: Sequence[int], pool_s
         grads.append(g.reshape(-1, d))
     if len(slots) == 1:  # one layer: its own tensors (views), no concatenated copies
         return merge_fetches(slots[0], weights[0], grads[0], pool_size, zero_padding, slot_counts)
-    return merge_fetches(torch.cat(slots), torch.cat(weights), torch.cat(grads), pool_size, zero_padding,
-                         slot_counts)
+    return merge_fetches(*_stacked(slots, weights, grads), pool_size, zero_padding, slot_counts)
 
 
 def fetched_row_grads(aux: Dict, probe_grads, layers: Sequence[int], pool_size: int):
