@@ -2,9 +2,10 @@
 config.py:9-61) around this library's MemoryPool.
 
 The backbone (embedding, attention, layer norms, feed-forward blocks, router
-and gated memory write-back) is small dense work and runs as plain torch ops
-in fp32; every memory read is MemoryPool (libmpl.so).  Parameter names and
-shapes follow the Flax modules, so a checkpoint of the reference
+and gated memory write-back) is small dense work: plain torch ops in fp32 in
+training, fused dense layers and causal attention (mpl_dense_layers,
+mpl_causal_attention) under torch.no_grad on the GPU; every memory read is
+MemoryPool (libmpl.so).  Parameter names and shapes follow the Flax modules, so a checkpoint of the reference
 (model_amd/checkpoint.py) loads into it:
 
   embed/embedding [vocab, d]            nn.Embed (logits use embed.attend)
