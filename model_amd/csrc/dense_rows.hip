@@ -22,9 +22,9 @@
 // 6 us of launch, first loads and epilogue around them and 5 us for LayerNorm.
 // A chunk takes 0.56 us at one wave a SIMD; 0.47 without the staging between
 // the MFMAs.  Measured, 4,096 rows, us, with one LDS buffer and one register
-// set -> now: K = 256, N = 768 with LayerNorm 30.5 -> 27.5, N = 1,024 with
-// LayerNorm and GELU 41.7 -> 36.8, N = 256 13.2 -> 11.5, K = 1,024, N = 256
-// 34.2 -> 25.9.  Chunks of 64 columns, 16x16x4 MFMAs and two groups of waves
+// set -> now: K = 256, N = 768 with LayerNorm 30.5 -> 27.1, N = 1,024 with
+// LayerNorm and GELU 41.7 -> 37.6, N = 256 13.2 -> 11.5, K = 1,024, N = 256
+// 34.2 -> 26.0.  Chunks of 64 columns, 16x16x4 MFMAs and two groups of waves
 // splitting K measured no faster.
 #include <math.h>
 
