@@ -26,7 +26,8 @@ __global__ __launch_bounds__(kGatherThreads) void gather_wsum_kernel(
     if (shuffle) sl = (int)(((int64_t)sl + N / 2 + 1) % N);
     sl = in ? (int)min(max((int64_t)sl, (int64_t)0), N - 1) : 0;  // out-of-range ids read the nearest row
     ww = in ? ww : 0.f;
-    acc.add_chunk(base, sl, ww, min(kWave, R - r0), lane);
+    if (R - r0 >= kWave) acc.add_chunk(base, sl, ww, kWave, lane);  // uniform
+    else acc.template add_chunk<true>(base, sl, ww, R - r0, lane);
   }
   acc.store(out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
 }

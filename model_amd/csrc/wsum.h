@@ -57,6 +57,13 @@ struct Vec16<float> {
   }
 };
 
+// Zeroes a loaded vector where !ok, by bits: a weight of 0 alone would make a
+// NaN of an infinite entry.
+__device__ __forceinline__ uint4 keep_if(uint4 u, bool ok) {
+  const uint32_t m = ok ? 0xFFFFFFFFu : 0u;
+  return make_uint4(u.x & m, u.y & m, u.z & m, u.w & m);
+}
+
 // VR = 16-byte vectors per row.  Either VR divides 64 (several rows per
 // instruction) or VR is a multiple of 64 (VR/64 vectors per lane per row).
 //
@@ -86,7 +93,9 @@ struct Wsum {
 
   // Adds rows 0..nr-1 of a chunk (nr <= 64): lane i holds row i's slot id
   // `sl` (already in [0, N)) and weight `ww`.  Batches of NB row groups: all
-  // NB loads are issued before any is used.
+  // NB loads are issued before any is used.  TAIL: nr < 64, what is loaded for
+  // rows past nr (any row of the table) is zeroed.
+  template <bool TAIL = false>
   __device__ __forceinline__ void add_chunk(const uint4* base, int sl, float ww, int nr, int lane) {
     const int sub = lane / LPR;
     const int col = lane % LPR;
@@ -98,12 +107,16 @@ struct Wsum {
       for (int b = 0; b < NB; ++b) {
         const bool ok = g0 + b < groups;
         const int row = ok ? (g0 + b) * RPI + sub : 0;  // rows past nr carry weight 0 and slot 0
+        const bool in = ok && row < nr;
         const int s = __shfl(sl, row);
         const float w = __shfl(ww, row);
         wv[b] = ok ? w : 0.f;
         const uint4* src = base + (int64_t)s * VR + col;
 #pragma unroll
-        for (int v = 0; v < VPL; ++v) buf[b][v] = NT ? load_nt(src + v * kWave) : src[v * kWave];
+        for (int v = 0; v < VPL; ++v) {
+          const uint4 u = NT ? load_nt(src + v * kWave) : src[v * kWave];
+          buf[b][v] = TAIL ? keep_if(u, in) : u;
+        }
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
@@ -186,7 +199,7 @@ struct WsumAny {
         wv[b] = ok && on ? w : 0.f;
         if (r0 + b * RPI < nr) {  // wave-uniform
           const uint4* src = base + (int64_t)s * VR + col;
-          buf[b] = NT ? load_nt(src) : *src;
+          buf[b] = keep_if(NT ? load_nt(src) : *src, ok);  // lanes past nr read row 0 again
         }
       }
 #pragma unroll

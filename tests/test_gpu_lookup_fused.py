@@ -120,3 +120,27 @@ def test_lookup_zero_tokens_and_errors(gpu_lib):
     rc = L.mpl_lookup(None, _lib.MPL_Q_RAW, None, None, 4, 4, 64, 64, 16, _lib.MPL_F16, None, None, None,
                       None, 0, None, None, None, None, None, None, 99, 256, 0, None, s)
     assert rc != 0 and b"values_dtype" in L.mpl_last_error()
+
+
+@pytest.mark.parametrize("H,k,d,vdt", [
+    (4, 5, 24, torch.float16),    # fused, 21 rows an instruction: the one load reaches a row past the last
+    (4, 7, 24, torch.float16),    # fused, a second load with 7 rows of 21
+    (4, 9, 64, torch.float32),    # fused, 4 rows an instruction, no row past the last
+    (2, 9, 24, torch.float16),    # the read alone, any width
+    (2, 9, 256, torch.float16),   # the read alone, 18 rows of a batch of 64
+    (1, 5, 128, torch.float32),   # the same, fp32
+    (8, 10, 512, torch.float16),  # 64 rows and 16 more
+])
+def test_infinite_entries_stay_infinite(gpu_lib, H, k, d, vdt):
+    """A table whose column 0 is +inf: every weight is positive, so that
+    column of the result is +inf, and the others are finite.  Rows past the
+    last one take no part in the sum, not even with weight 0."""
+    from model_amd.memory import MemoryPool
+    pool = MemoryPool(32, H, 32, d, k, values_dtype=vdt)
+    params = pool.init(0)
+    params["params"]["values"][:, 0] = float("inf")
+    q = torch.randn((37, H, 32), generator=torch.Generator(device="cuda").manual_seed(k), device="cuda")
+    res = pool.lookup(params["params"], q)
+    assert float(res["weights"].min()) > 0
+    assert torch.equal(res["out"][:, 0], torch.full((37,), float("inf"), device="cuda"))
+    assert bool(torch.isfinite(res["out"][:, 1:]).all())
