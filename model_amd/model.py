@@ -538,9 +538,11 @@ class MemoryPoolLM:
                 logits = F.linear(_ln(x, lf), emb)[:, None]
         return logits, _LazyMerged(layer_aux)
 
-    def _fused_forward_ok(self, p, tokens) -> bool:
+    def _fused_forward_ok(self, p, tokens, pool_off: bool = False) -> bool:
         """Whether _forward_gpu computes this call: plain inference on the
-        GPU with fp32 parameters whose widths the fused kernels take."""
+        GPU with fp32 parameters whose widths the fused kernels take.  Looks
+        only at the parameters that the call reads (with pool_off the memory
+        layers' own may be missing)."""
         cfg = self.cfg
         d, H = cfg.d_model, cfg.n_heads
         if (not tokens.is_cuda or type(tokens) is not torch.Tensor or tokens.numel() == 0 or not _plain_inference()
@@ -559,7 +561,7 @@ class MemoryPoolLM:
             mem = self.pool is not None and i in cfg.memory_layers
             names += [f"ln_attn_{i}", f"attn_{i}", f"ln_ffn_{i}"]
             names += [f"ffn_in_{i}", f"ffn_out_{i}"] if not mem or cfg.memory_ffn else []
-            names += [f"router_{i}", f"mem_gate_{i}", f"mem_out_{i}"] if mem else []
+            names += [f"router_{i}", f"mem_gate_{i}", f"mem_out_{i}"] if mem and not pool_off else []
         emb, pe = p["embed"]["embedding"], p["pos_embed"]
         return plain(emb) and plain(pe) and emb.shape[0] % 4 == 0 and all(plain(p[nm]) for nm in names)
 
@@ -646,7 +648,7 @@ class MemoryPoolLM:
                 and not pool_off and not route_through_pool and probes is None and not shuffle_pool):
             return self._decode_step_gpu(p, tokens, positions, cache, noise_scale, rngs, input_rows)
         if (not self.decode and positions is None and not train and not route_through_pool and probes is None
-                and not sparse_grad and self._fused_forward_ok(p, tokens)):
+                and not sparse_grad and self._fused_forward_ok(p, tokens, pool_off)):
             return self._forward_gpu(p, tokens, pool_off, noise_scale, shuffle_pool, rngs)
         emb = p["embed"]["embedding"]
         if positions is None:

@@ -131,3 +131,23 @@ def test_fused_forward_equals_general_path(gpu_lib, B, T, heads, memory_ffn, use
     # transforms and modes take the general path
     with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
         assert not model._fused_forward_ok(params["params"], tokens)
+
+
+def _small_model(**kw):
+    cfg = ModelConfig(**{**dict(vocab_size=400, max_len=80, d_model=128, n_layers=2, n_heads=2, ffn_mult=2,
+                                use_memory=True, memory_layers=(1,), memory_ffn=True, n_sub_keys=24, pool_heads=2,
+                                d_key=32, d_value=64, top_k=8, values_dtype=torch.float32), **kw})
+    model = MemoryPoolLM(cfg)
+    tokens = torch.randint(0, cfg.vocab_size, (2, 33), generator=torch.Generator().manual_seed(2)).cuda()
+    return model, model.init(4), tokens
+
+
+def test_pool_off_without_memory_parameters(gpu_lib):
+    """pool_off reads no parameter of the memory layers: they may be missing."""
+    model, params, tokens = _small_model()
+    want = model.apply(params, tokens, pool_off=True)[0].detach()  # gradients enabled: the general path
+    bare = {k: v for k, v in params["params"].items() if k not in ("router_1", "mem_gate_1", "mem_out_1", "pool")}
+    with torch.no_grad():
+        assert model._fused_forward_ok(bare, tokens, True)
+        got, aux = model.apply({"params": bare}, tokens, pool_off=True)
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
