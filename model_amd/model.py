@@ -550,20 +550,44 @@ class MemoryPoolLM:
                 or tokens.numel() > 65535 * 64 or cfg.pool_heads * cfg.d_key % 4 or cfg.d_value % 4):
             return False
 
-        def plain(t):
-            if isinstance(t, dict):
-                return all(plain(v) for v in t.values())
-            return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_contiguous()
-                    and t.device == tokens.device and t.data_ptr() % 16 == 0)
+        dev = tokens.device
 
-        names = ["ln_final"]
+        def plain(t):
+            return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_contiguous()
+                    and t.device == dev and t.data_ptr() % 16 == 0)
+
+        # Of exactly the shapes that the general path's products take: a shape
+        # that it broadcasts or refuses is left to it (the fused launches read
+        # a kernel by its address and number of elements alone).
+        def dense(w, K, N):
+            return (plain(w["kernel"]) and w["kernel"].shape == (K, N) and plain(w["bias"])
+                    and w["bias"].shape == (N,))
+
+        def ln(w):
+            return plain(w["scale"]) and w["scale"].shape == (d,) and plain(w["bias"]) and w["bias"].shape == (d,)
+
+        def attention(a):  # the general path reshapes these itself
+            return (all(plain(w["kernel"]) and w["kernel"].numel() == d * d and plain(w["bias"])
+                        for w in (a["query"], a["key"], a["value"], a["out"]))
+                    and all(a[nm]["bias"].numel() == d for nm in ("query", "key", "value"))
+                    and a["out"]["bias"].shape == (d,))
+
         for i in range(cfg.n_layers):
             mem = self.pool is not None and i in cfg.memory_layers
-            names += [f"ln_attn_{i}", f"attn_{i}", f"ln_ffn_{i}"]
-            names += [f"ffn_in_{i}", f"ffn_out_{i}"] if not mem or cfg.memory_ffn else []
-            names += [f"router_{i}", f"mem_gate_{i}", f"mem_out_{i}"] if mem and not pool_off else []
+            if not (ln(p[f"ln_attn_{i}"]) and attention(p[f"attn_{i}"]) and ln(p[f"ln_ffn_{i}"])):
+                return False
+            if not mem or cfg.memory_ffn:
+                fi, fo = p[f"ffn_in_{i}"], p[f"ffn_out_{i}"]
+                width = fi["bias"].numel()  # the parameters' own, whatever cfg.ffn_mult says
+                if width < 4 or width % 4 or not (dense(fi, d, width) and dense(fo, width, d)):
+                    return False
+            if mem and not pool_off and not (dense(p[f"router_{i}"], d, cfg.pool_heads * cfg.d_key)
+                                             and dense(p[f"mem_gate_{i}"], d, cfg.d_value)
+                                             and dense(p[f"mem_out_{i}"], cfg.d_value, d)):
+                return False
         emb, pe = p["embed"]["embedding"], p["pos_embed"]
-        return plain(emb) and plain(pe) and emb.shape[0] % 4 == 0 and all(plain(p[nm]) for nm in names)
+        return (plain(emb) and emb.dim() == 2 and emb.shape[1] == d and emb.shape[0] % 4 == 0
+                and plain(pe) and pe.dim() == 2 and pe.shape[1] == d and ln(p["ln_final"]))
 
     def _forward_gpu(self, p, tokens, pool_off, noise_scale, shuffle_pool, rngs):
         """The general path of apply() for plain inference over whole

@@ -151,3 +151,36 @@ def test_pool_off_without_memory_parameters(gpu_lib):
         assert model._fused_forward_ok(bare, tokens, True)
         got, aux = model.apply({"params": bare}, tokens, pool_off=True)
     torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
+
+
+def test_shapes_the_general_path_refuses_stay_refused(gpu_lib):
+    """A kernel of the right number of elements in another shape (saved as
+    [out, in], say) is an error, not a product with its elements in another
+    order."""
+    for name, shape in (("ffn_in_0", (256, 128)), ("ffn_out_1", (128, 256)), ("router_1", (128, 2, 32)),
+                        ("mem_gate_1", (64, 128)), ("mem_out_1", (128, 64))):
+        model, params, tokens = _small_model()
+        params["params"][name]["kernel"] = params["params"][name]["kernel"].reshape(shape)
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            model.apply(params, tokens)
+    for part in ("scale", "bias"):
+        model, params, tokens = _small_model()
+        params["params"]["ln_ffn_0"][part] = params["params"]["ln_ffn_0"][part][None]
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            model.apply(params, tokens)
+
+
+def test_shapes_the_general_path_broadcasts_are_taken(gpu_lib):
+    """A gate of one column, biases of one element and a hidden layer whose
+    width is no multiple of 4: accepted, with the general path's result."""
+    model, params, tokens = _small_model()
+    p = params["params"]
+    g = torch.Generator(device="cuda").manual_seed(7)
+    p["mem_gate_1"] = {"kernel": p["mem_gate_1"]["kernel"][:, :1].contiguous(), "bias": p["mem_gate_1"]["bias"][:1]}
+    p["ffn_out_1"]["bias"] = torch.randn(1, generator=g, device="cuda")
+    p["ffn_in_0"] = {"kernel": p["ffn_in_0"]["kernel"][:, :250].contiguous(), "bias": p["ffn_in_0"]["bias"][:250]}
+    p["ffn_out_0"]["kernel"] = p["ffn_out_0"]["kernel"][:250]
+    want = model.apply(params, tokens)[0].detach()
+    with torch.no_grad():
+        got = model.apply(params, tokens)[0]
+    torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4)
