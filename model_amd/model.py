@@ -552,9 +552,9 @@ class MemoryPoolLM:
 
         dev = tokens.device
 
-        def plain(t):
+        def plain(t, align=16):
             return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float32 and t.is_contiguous()
-                    and t.device == dev and t.data_ptr() % 16 == 0)
+                    and t.device == dev and t.data_ptr() % align == 0)
 
         # Of exactly the shapes that the general path's products take: a shape
         # that it broadcasts or refuses is left to it (the fused launches read
@@ -585,9 +585,10 @@ class MemoryPoolLM:
                                              and dense(p[f"mem_gate_{i}"], d, cfg.d_value)
                                              and dense(p[f"mem_out_{i}"], cfg.d_value, d)):
                 return False
+        # the tables are read by torch's own indexing and product: any vocabulary
         emb, pe = p["embed"]["embedding"], p["pos_embed"]
-        return (plain(emb) and emb.dim() == 2 and emb.shape[1] == d and emb.shape[0] % 4 == 0
-                and plain(pe) and pe.dim() == 2 and pe.shape[1] == d and ln(p["ln_final"]))
+        return (plain(emb, 4) and emb.dim() == 2 and emb.shape[1] == d
+                and plain(pe, 4) and pe.dim() == 2 and pe.shape[1] == d and ln(p["ln_final"]))
 
     def _forward_gpu(self, p, tokens, pool_off, noise_scale, shuffle_pool, rngs):
         """The general path of apply() for plain inference over whole
