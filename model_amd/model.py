@@ -252,6 +252,29 @@ def _plain_inference() -> bool:
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
 
 
+def _fused_forward_pays(d: int, heads: int, batch: int, length: int) -> bool:
+    """Whether the fused launches are the faster way through a backbone of
+    width d: mpl_dense_layers reaches 60 to 82 TFLOP/s, the library's product
+    up to 120, the more the wider it is; so a token loses about d^3 in the
+    dense layers and wins heads * length in the attention (no score matrix),
+    and few tokens win 150 us a layer of launches.  Measured, 2 layers, ffn
+    4 d, us fused / general, heads of 64 and of 128:
+      d = 896:    64 x 256: 6,851 / 6,838 and 6,966 / 6,494; none of 22
+                  other shapes slower (16 x 512: 3,597 / 4,073, 3,635 / 3,730)
+      d = 1,024:  1 x 256: 416 / 531;  8 x 128: 660 / 707;  16 x 256: 2,265 /
+                  2,223 and 2,263 / 2,194;  64 x 256: 8,772 / 8,281 and 8,834 /
+                  7,874;  16 x 512: 4,555 / 4,767 and 4,512 / 4,355;
+                  16 x 1,024: 10,007 / 11,155 and 9,941 / 9,617
+      d = 1,280:  1 x 128: 480 / 526;  16 x 64: 1,082 / 956;
+                  16 x 1,024: 15,052 / 15,608 and 15,016 / 13,703
+      d = 2,048:  1 x 16: 708 / 556;  16 x 256: 8,268 / 6,935;
+                  4 x 1,024: 8,874 / 8,485;  2 x 2,048: 9,377 / 10,491;
+                  1 x 4,096: 10,306 / 14,421 (heads of 64)."""
+    tokens = batch * length
+    return (d <= 896 or d * d * (d // heads) <= 150_000 * length
+            or tokens <= (1024 if d <= 1024 else 128 if d <= 1280 else 0))
+
+
 def decode_attention(qkv: torch.Tensor, positions: torch.Tensor, layer_cache: Dict[str, torch.Tensor], heads: int,
                      scale: float) -> torch.Tensor:
     """mpl_decode_attention: qkv [B, 3 * heads * hd] fp32 (query, key and
@@ -547,7 +570,8 @@ class MemoryPoolLM:
         d, H = cfg.d_model, cfg.n_heads
         if (not tokens.is_cuda or type(tokens) is not torch.Tensor or tokens.numel() == 0 or not _plain_inference()
                 or d % 4 or d % H or d // H not in (32, 64, 128) or tokens.shape[0] * H > 65535
-                or tokens.numel() > 65535 * 64 or cfg.pool_heads * cfg.d_key % 4 or cfg.d_value % 4):
+                or tokens.numel() > 65535 * 64 or cfg.pool_heads * cfg.d_key % 4 or cfg.d_value % 4
+                or not _fused_forward_pays(d, H, *tokens.shape)):
             return False
 
         dev = tokens.device

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from model_amd import _lib
-from model_amd.model import MemoryPoolLM, ModelConfig, causal_attention, dense_layers
+from model_amd.model import MemoryPoolLM, ModelConfig, _fused_forward_pays, causal_attention, dense_layers
 from oracle import backbone as ob
 
 pytestmark = pytest.mark.gpu
@@ -207,3 +207,15 @@ def test_any_vocabulary(gpu_lib, vocab, dtype):
     assert bool(same.all()) if dtype == torch.float32 else float(same.float().mean()) > 0.8
     tol = 1e-4 if dtype == torch.float32 else 2e-3
     torch.testing.assert_close(got[same], want.detach()[same], rtol=tol, atol=tol)
+
+
+def test_wide_short_calls_take_the_general_path(gpu_lib):
+    """At widths where the library's products are faster than the fused ones
+    only calls that win it back (long sequences, few tokens) are fused."""
+    model, params, tokens = _small_model(d_model=2048, n_heads=32, n_layers=1, ffn_mult=1, memory_layers=())
+    with torch.no_grad():
+        assert not model._fused_forward_ok(params["params"], tokens)
+    pays = [(128, 4, 64, 4096), (896, 7, 16, 512), (1024, 16, 1, 1024), (1024, 16, 16, 512), (1280, 20, 1, 128),
+            (2048, 32, 2, 2048)]
+    costs = [(1024, 8, 64, 256), (1280, 10, 16, 64), (1280, 10, 16, 1024), (2048, 32, 1, 16), (2048, 32, 4, 1024)]
+    assert all(_fused_forward_pays(*c) for c in pays) and not any(_fused_forward_pays(*c) for c in costs)
