@@ -26,6 +26,7 @@ elimination for the same effect, memory.py:215).
 
 from __future__ import annotations
 
+import functools
 import math
 from typing import Any, Dict, Optional, Tuple
 
@@ -167,16 +168,46 @@ class _Views(dict):
 
 
 class _Result(dict):
-    """The lookup's result; keys it does not hold are its _Views (shared with
-    the aux, which refers to them and not to this dict: no reference cycle
-    keeps a call's tensors until a garbage collection)."""
+    """The lookup's result.  A key of its _Views (shared with the aux, which
+    refers to them and not to this dict: no reference cycle keeps a call's
+    tensors until a garbage collection) enters the dict when it is read, and
+    all of them do before anything that looks at more than one key (``in``,
+    ``get``, ``keys``, iteration, copies); "q_hat" only when it is read."""
 
     def __init__(self, eager: Dict[str, Any], views: _Views):
         super().__init__(eager)
         self._views = views
+        self._pending = set(views._make)
 
     def __missing__(self, key):
-        return self._views[key]
+        if key not in self._pending and key != "q_hat":
+            raise KeyError(key)
+        self._pending.discard(key)
+        v = self[key] = self._views[key]
+        return v
+
+    def _fill(self):
+        for key in [k for k in self._views._make if k in self._pending]:
+            if not dict.__contains__(self, key):  # else it was set by the caller
+                self[key]
+        self._pending.clear()
+
+
+def _filled(name: str):
+    method = getattr(dict, name)
+
+    @functools.wraps(method)
+    def call(self, *args, **kw):
+        self._fill()
+        return method(self, *args, **kw)
+
+    return call
+
+
+for _name in ("__contains__", "__delitem__", "__eq__", "__ior__", "__iter__", "__len__", "__ne__", "__or__",
+              "__repr__", "__reversed__", "__ror__", "clear", "copy", "get", "items", "keys", "pop", "popitem",
+              "setdefault", "values"):
+    setattr(_Result, _name, _filled(_name))
 
 
 def routing_seed(rngs: Optional[Dict[str, Any]]) -> int:
