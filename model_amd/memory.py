@@ -186,6 +186,13 @@ class _Result(dict):
         v = self[key] = self._views[key]
         return v
 
+    def for_backward(self) -> "_Result":
+        """What _lookup_backward reads, without the output, the aux and the
+        noise: an autograd node that kept its own output would be a reference
+        cycle, and the noise ([M, H, 2, n]) is not read again."""
+        return _Result({k: self[k] for k in ("q_len", "k_hat", "packed", "score_code", "temperature", "staged")},
+                       self._views)
+
     def _fill(self):
         for key in [k for k in self._views._make if k in self._pending]:
             if not dict.__contains__(self, key):  # else it was set by the caller
@@ -737,7 +744,7 @@ class _LookupFunction(torch.autograd.Function):
                           shuffle_reads=opts["shuffle_reads"], rngs=opts["rngs"])
         aux = res["aux"]
         balance = aux["balance_loss"]  # also computes f and p (memory.py:196-213)
-        ctx.pool, ctx.opts, ctx.res = pool, opts, res
+        ctx.pool, ctx.opts, ctx.res = pool, opts, res.for_backward()
         ctx.internal = aux.internal
         opts["_aux"] = aux  # handed back to the caller with the differentiable balance loss
         ctx.shapes = (tuple(queries.shape), queries.dtype, sub_keys.dtype, log_temperature.dtype)
