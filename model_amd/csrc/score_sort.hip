@@ -17,9 +17,9 @@
 //
 // This file is compiled without IEEE mode and NaN handling of min / max (no
 // canonicalisation of the keys, which the compiler would otherwise add to
-// every value it cannot trace: +25% double-precision instructions).  NaN scores
-// are turned into -FLT_MAX by a v_max before they become keys (no cosine is
-// that small; the output takes it for "none"), so no key is a NaN.
+// every value it cannot trace: +28% double-precision instructions).  NaN scores
+// are turned into -FLT_MAX, by their bits, before they become keys (no cosine
+// is that small; the output takes it for "none"), so no key is a NaN.
 #include <float.h>
 
 #include "score_stage1.h"
@@ -67,13 +67,31 @@ __global__ __launch_bounds__(kWave, 2) void score_sort_kernel(ScoreParams p) {
     }
     return x;
   };
-  // The lane's keys of block b, sorted.  MFMA sums start at +0, so no score
-  // is -0; below a negative score the index is stored uncomplemented (topk.h).
+  // NaN scores of a block become -FLT_MAX, by integer operations on their
+  // bits: the compiler takes every float of this file for a number.  Cosines
+  // are below 2, so one test of the bits of all 16 (bit 30: 2 and above, inf
+  // and NaN) decides for the wave whether any has to be looked at.
+  auto drop_nans = [&](f32x16& x) __attribute__((always_inline)) {
+    asm("" : "+v"(x));  // no assumption about the MFMAs' results passes here
+    uint32_t any = 0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) any |= __float_as_uint(x[r]);
+    if (__ballot((any & 0x40000000u) != 0) != 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t u = __float_as_uint(x[r]);
+        x[r] = __uint_as_float((u & 0x7FFFFFFFu) > 0x7F800000u ? 0xFF7FFFFFu : u);
+      }
+    }
+  };
+  // The lane's keys of block b, sorted.  MFMA sums start at +0, so a score is
+  // -0 only where its exact value is negative and underflows; below a negative
+  // score the index is stored uncomplemented (topk.h).
   auto sorted_keys = [&](int b, const f32x16& x, Key (&c)[16]) __attribute__((always_inline)) {
     const uint32_t nidx = ~(uint32_t)(b * 32 + 4 * par);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const uint32_t hi = __float_as_uint(__builtin_fmaxf(x[r], -FLT_MAX));
+      const uint32_t hi = __float_as_uint(x[r]);
       c[r] = key_of(hi, (nidx - (uint32_t)(8 * (r >> 2) + (r & 3))) ^ (uint32_t)((int)hi >> 31));
     }
     if (b * 32 + 32 > p.n) {  // wave-uniform: only the last block can hold padded keys
@@ -92,6 +110,7 @@ __global__ __launch_bounds__(kWave, 2) void score_sort_kernel(ScoreParams p) {
     // the next block's MFMAs beside this block's sort; past the end they
     // score the last block again and nobody reads them
     for (int b = b_begin; b < b_end; ++b) {
+      drop_nans(x);
       const f32x16 y = score(b + 2);
       sorted_keys(b, x, c);
       if (b == b_begin) {  // wave-uniform: the list is empty
@@ -106,6 +125,7 @@ __global__ __launch_bounds__(kWave, 2) void score_sort_kernel(ScoreParams p) {
     // fp32 MFMAs take longer than the sort: none is issued for nothing
     for (int b = b_begin; b < b_end; ++b) {
       if (b > b_begin) x = score(b + 1);
+      drop_nans(x);
       sorted_keys(b, x, c);
       if (b == b_begin) {
 #pragma unroll

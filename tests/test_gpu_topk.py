@@ -272,3 +272,48 @@ def test_sorted_stage1_equals_thresholds(gpu_lib, M, n, half, k, score, bad):
     assert bad or int(got[0][0].min()) >= 0
     if bad:
         assert (got[0][0][1::3, 0, 1] == -1).all()
+
+
+@pytest.mark.parametrize("M,n,k,nan_bits,scale", [
+    (40, 300, 16, 0x7FC00000, 1.0),    # the usual quiet NaN
+    (40, 300, 32, 0xFFC00000, 1.0),    # negative
+    (33, 100, 9, 0x7F800001, 1.0),     # signalling, smallest payload
+    (33, 100, 16, 0xFFFFFFFF, 1.0),    # all ones: its bits would make a key that is no number
+    (64, 70, 16, None, 300.0),         # no NaN, scores of 2 and above
+    (64, 70, 16, 0x7FFFFFFF, 1e30),    # both, scores up to 1e31
+])
+def test_sorted_stage1_nan_bits_and_large_scores(gpu_lib, M, n, k, nan_bits, scale):
+    """Queries read as they are (MPL_Q_NORMALIZED, fp32 scoring): NaN of any
+    bits is never selected, and scores past the range of cosines order as any
+    others; equal to stage 1 by thresholds (zero noise) bit for bit."""
+    L = _lib.lib()
+    H, half, score = 2, 16, _lib.MPL_F32
+    g = torch.Generator().manual_seed(n + k)
+    q = torch.nn.functional.normalize(torch.randn((M, H, 2, half), generator=g), dim=-1) * scale
+    keys = torch.randn((H, 2, n, half), generator=g).cuda()
+    if nan_bits is not None:
+        q.view(torch.int32)[::3, 1, 0, 5] = nan_bits - (1 << 32) if nan_bits >> 31 else nan_bits
+    q = q.cuda()
+    packed = torch.empty(L.mpl_packed_keys_bytes(H, n, half, score), dtype=torch.uint8, device="cuda")
+    st = _lib.stream_ptr(q.device)
+    _lib.check(L.mpl_pack_keys(_lib.ptr(keys), H, n, half, score, None, _lib.ptr(packed), st), "pack")
+    one, zero = torch.ones(1, device="cuda"), torch.zeros(1, device="cuda")
+    no_noise = torch.zeros((M, H, 2, n), device="cuda")
+    wsb = L.mpl_score_topk_workspace_bytes(M, H, n, half, k)
+    got = []
+    for gum in (None, no_noise):
+        ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+        ids = torch.full((M, H, 2, k), -7, dtype=torch.int32, device="cuda")
+        sc = torch.full((M, H, 2, k), 7.0, device="cuda")
+        _lib.check(L.mpl_score_topk(_lib.ptr(q), _lib.MPL_Q_NORMALIZED, None, _lib.ptr(packed), M, H, n, half, k,
+                                    score, _lib.ptr(one), _lib.ptr(gum), _lib.ptr(zero if gum is not None else None),
+                                    _lib.ptr(ws), wsb, _lib.ptr(ids), _lib.ptr(sc), st), "topk")
+        torch.cuda.synchronize()
+        got.append((ids.cpu().numpy(), sc.cpu().numpy()))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    if nan_bits is not None:
+        assert (got[0][0][::3, 1, 0] == -1).all()
+    rest = np.ones((M, H, 2), bool)
+    rest[::3, 1, 0] = nan_bits is None
+    assert (got[0][0][rest] >= 0).all()
