@@ -177,12 +177,12 @@ class _Result(dict):
     def __init__(self, eager: Dict[str, Any], views: _Views):
         super().__init__(eager)
         self._views = views
-        self._pending = set(views._make)
+
+    _full = False  # whether all the views have entered
 
     def __missing__(self, key):
-        if key not in self._pending and key != "q_hat":
+        if self._full and key != "q_hat":  # the caller took it out
             raise KeyError(key)
-        self._pending.discard(key)
         v = self[key] = self._views[key]
         return v
 
@@ -194,10 +194,11 @@ class _Result(dict):
                        self._views)
 
     def _fill(self):
-        for key in [k for k in self._views._make if k in self._pending]:
-            if not dict.__contains__(self, key):  # else it was set by the caller
-                self[key]
-        self._pending.clear()
+        if not self._full:
+            for key in self._views._make:
+                if not dict.__contains__(self, key):  # else it was read, or set by the caller
+                    self[key]
+            self._full = True
 
 
 def _filled(name: str):
