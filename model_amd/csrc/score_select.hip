@@ -546,7 +546,9 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
   // below it, so each position ends with its largest positive score, or -inf
   // if it saw none.  Either way the 32 values of a lane pair (one query) are
   // scores of distinct keys or -inf, so their k-th largest is a lower bound
-  // on that query's k-th best score; negative scores only loosen it.
+  // on that query's k-th best score; negative scores only loosen it.  A NaN
+  // (of a NaN key) beats the scores of its position, or -inf, by its bits; it
+  // counts as -inf after the pass.
   int ma[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) ma[r] = (int)0xff800000u;  // -inf
@@ -588,7 +590,10 @@ __global__ __launch_bounds__(kScoreThreads, (stage1_min_waves<T, NOISE, KMAX>())
   }
   float fa[16];  // own maxima
 #pragma unroll
-  for (int r = 0; r < 16; ++r) fa[r] = __int_as_float(ma[r]);
+  for (int r = 0; r < 16; ++r) {
+    const float v = __int_as_float(ma[r]);
+    fa[r] = v == v ? v : -INFINITY;
+  }
   float bound;
   if constexpr (KMAX == 16) {
     bound = kth_of_pair16(fa, par, p.k);

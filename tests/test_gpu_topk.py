@@ -317,3 +317,41 @@ def test_sorted_stage1_nan_bits_and_large_scores(gpu_lib, M, n, k, nan_bits, sca
     rest = np.ones((M, H, 2), bool)
     rest[::3, 1, 0] = nan_bits is None
     assert (got[0][0][rest] >= 0).all()
+
+
+@pytest.mark.parametrize("M,n,half,k,score,noise", [
+    (8192, 300, 128, 32, _lib.MPL_F16, False),
+    (8192, 512, 128, 16, _lib.MPL_F16, False),
+    (4096, 8192, 128, 16, _lib.MPL_F16, False),
+    (4096, 8192, 64, 9, _lib.MPL_F32, False),
+    (2000, 300, 64, 32, _lib.MPL_F32, True),
+    (2000, 300, 64, 16, _lib.MPL_F16, True),
+])
+@pytest.mark.parametrize("nan_bits", [0x7FC00000, 0xFFC00000])
+def test_nan_keys_leave_the_others_alone(gpu_lib, M, n, half, k, score, noise, nan_bits):
+    """NaN keys are never selected and change nothing for the others: the same
+    ids and scores as with zeros in their place, whose score of 0 lies below
+    the k best of these keys."""
+    L = _lib.lib()
+    H = 4
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    q = torch.randn((M, H, 2, half), generator=g, device="cuda")
+    keys = torch.randn((H, 2, n, half), generator=g, device="cuda")
+    st = _lib.stream_ptr(q.device)
+    one, zero = torch.ones(1, device="cuda"), torch.zeros(1, device="cuda")
+    gum = torch.zeros((M, H, 2, n), device="cuda") if noise else None
+    wsb = L.mpl_score_topk_workspace_bytes(M, H, n, half, k)
+    got = []
+    for bits in (nan_bits, 0):
+        keys.view(torch.int32)[:, :, 4::37] = bits - (1 << 32) if bits >> 31 else bits
+        packed = torch.empty(L.mpl_packed_keys_bytes(H, n, half, score), dtype=torch.uint8, device="cuda")
+        _lib.check(L.mpl_pack_keys(_lib.ptr(keys), H, n, half, score, None, _lib.ptr(packed), st), "pack")
+        ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+        ids = torch.full((M, H, 2, k), -7, dtype=torch.int32, device="cuda")
+        sc = torch.full((M, H, 2, k), 7.0, device="cuda")
+        _lib.check(L.mpl_score_topk(_lib.ptr(q), _lib.MPL_Q_RAW, None, _lib.ptr(packed), M, H, n, half, k, score,
+                                    _lib.ptr(one), _lib.ptr(gum), _lib.ptr(zero if noise else None), _lib.ptr(ws), wsb,
+                                    _lib.ptr(ids), _lib.ptr(sc), st), "topk")
+        got.append((ids, sc))
+    assert bool((got[1][1] > 0).all())  # the zero keys are not among them
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
