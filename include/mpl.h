@@ -109,6 +109,19 @@ int mpl_score_select(const void* queries, int query_mode, float* q_len, const vo
                      int32_t* slots, float* weights, void* stream);
 
 /*
+ * No counterpart in the reference: the stage-1 kernel that a selection of
+ * these sizes takes (MPL_STAGE1_*: for up to 4 tokens, by sorting, by
+ * thresholds), and into how many splits of how many blocks of 32 keys its key
+ * range goes (either pointer may be NULL).  noise: with a gumbel tensor; pair:
+ * mpl_score_select and mpl_lookup (1) or mpl_score_topk (0).  On the host
+ * only; -1 for sizes that those calls refuse.  The choice is a matter of time
+ * and never of results.
+ */
+enum { MPL_STAGE1_DECODE = 0, MPL_STAGE1_SORT = 1, MPL_STAGE1_THRESHOLDS = 2 };
+int mpl_score_plan(int64_t M, int H, int n, int half, int k, int score_dtype, int noise, int pair, int* splits,
+                   int* blocks_per_split);
+
+/*
  * memory.py:132-193 (MemoryPool.__call__'s forward read, model.py:112-113):
  * mpl_score_select followed by the value read of mpl_gather_wsum, in one
  * call.  Same arguments, workspace (mpl_score_select_workspace_bytes) and

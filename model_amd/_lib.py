@@ -17,6 +17,7 @@ MPL_OK, MPL_EINVAL, MPL_EHIP, MPL_EWORKSPACE, MPL_EUNSUPPORTED = 0, 1, 2, 3, 4  
 MPL_Q_NORMALIZED, MPL_Q_RAW, MPL_Q_RAW_SCALED = 0, 1, 2
 MPL_ACT_NONE, MPL_ACT_GELU_TANH, MPL_ACT_SILU = 0, 1, 2
 MPL_W_IN_OUT, MPL_W_OUT_IN = 0, 1
+MPL_STAGE1_DECODE, MPL_STAGE1_SORT, MPL_STAGE1_THRESHOLDS = 0, 1, 2
 
 # name -> (restype, argtypes); the C ABI of include/mpl.h
 _P, _I, _I64, _F, _SZ = C.c_void_p, C.c_int, C.c_int64, C.c_float, C.c_size_t
@@ -51,6 +52,7 @@ SIGNATURES = {
     "mpl_scatter_rows": (_I, [_P, _P, _I64, _P, _I, _I64, _P, _P]),
     "mpl_copy_arrays": (_I, [_P, _P, _P, _I, _P]),
     "mpl_host_device_pointer": (_I, [_P, C.POINTER(C.c_void_p)]),
+    "mpl_score_plan": (_I, [_I64, _I, _I, _I, _I, _I, _I, _I, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "mpl_score_topk_workspace_bytes": (_SZ, [_I64, _I, _I, _I, _I]),
     "mpl_score_topk": (_I, [_P, _I, _P, _P, _I64, _I, _I, _I, _I, _I, _P, _P, _P, _P, _SZ, _P, _P, _P]),
     "mpl_merge_rows_workspace_bytes": (_SZ, [_I64, _I, _I64]),

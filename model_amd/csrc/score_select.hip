@@ -1711,6 +1711,14 @@ static Plan make_decode_plan(int n) {
   return pl;
 }
 
+// The plan a call takes; *decode: stage 1 is score_topk_decode.
+static Plan choose_plan(int64_t M, int H, int n, int half, int k, int score_dtype, bool noise, bool pair,
+                        bool* decode) {
+  *decode = !noise && score_dtype == MPL_F16 && decode_shape(M, k);
+  return *decode ? make_decode_plan(n) : noise ? make_plan(M, H, n, k)
+                                     : make_clean_plan(M, H, n, k, score_dtype, padded_half(half, score_dtype), pair);
+}
+
 // Workspace: the select scores with noise; per-split lists when split, and
 // for k <= 16 the lists of each reduction level (8 lists into one) until at
 // most 8 remain for stage 2.
@@ -1835,6 +1843,22 @@ extern "C" size_t mpl_score_topk_workspace_bytes(int64_t M, int H, int n, int ha
 // 2 and the softmax as well.  Without `pair`, flat_idx/slots/weights are null.
 // The value read fused into stage 2 (pair_read_k16), when the shapes allow:
 // returns false (nothing launched) otherwise.
+extern "C" int mpl_score_plan(int64_t M, int H, int n, int half, int k, int score_dtype, int noise, int pair,
+                              int* splits, int* blocks_per_split) {
+  clear_error();
+  if (M <= 0 || H <= 0 || k <= 0 || n < k || k > 32 || half <= 0 || half > 128 ||
+      (score_dtype != MPL_F32 && (score_dtype != MPL_F16 || half % 8 != 0))) {
+    set_error("mpl_score_plan: no plan for M=%lld H=%d n=%d half=%d k=%d score_dtype=%d", (long long)M, H, n, half, k,
+              score_dtype);
+    return -1;
+  }
+  bool decode;
+  const Plan pl = choose_plan(M, H, n, half, k, score_dtype, noise != 0, pair != 0, &decode);
+  if (splits != nullptr) *splits = pl.splits;
+  if (blocks_per_split != nullptr) *blocks_per_split = pl.blk_per_split;
+  return decode ? MPL_STAGE1_DECODE : pl.sort ? MPL_STAGE1_SORT : MPL_STAGE1_THRESHOLDS;
+}
+
 struct LookupRead {
   const void* values;
   int dtype;  // MPL_F16 or MPL_F32
@@ -1976,10 +2000,9 @@ static int select_impl(const char* who, bool pair, const void* queries, int quer
   MPL_REQUIRE(query_mode == MPL_Q_NORMALIZED || query_mode == MPL_Q_RAW || query_mode == MPL_Q_RAW_SCALED,
               MPL_EINVAL, "%s: bad query_mode %d", who, query_mode);
   const bool noise = gumbel != nullptr;
-  const bool decode = !noise && score_dtype == MPL_F16 && decode_shape(M, k);
+  bool decode;
+  const Plan pl = choose_plan(M, H, n, half, k, score_dtype, noise, pair, &decode);
   const int HP = padded_half(half, score_dtype);
-  const Plan pl = decode ? make_decode_plan(n) : noise ? make_plan(M, H, n, k)
-                                       : make_clean_plan(M, H, n, k, score_dtype, HP, pair);
   const size_t sel_need = ws_bytes(pl, M, H, k, noise);
   const size_t extra = pair ? 0 : topk_extra_bytes(pl, M, H, k);
   const size_t extra_at = (sel_need + 255) / 256 * 256;

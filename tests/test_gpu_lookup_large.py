@@ -2,10 +2,12 @@
 
 * 67,108,864 fp16 slots (n_sub_keys = 8,192, H = 4, d_key = 256, k = 16,
   d_value = 256; a 34 GB table in HBM) at 1, 16, 256 and 4,096 decode tokens.
-  These take every plan the selection has at that width: 64 short splits of
-  4 key blocks reduced by pair_wide_k16 (1 and 16 tokens), 32 splits of 8
-  blocks (256 tokens), and 2 splits of 128 blocks whose stage 2 is fused with
-  the value read (pair_read_k16, 4,096 tokens).
+  These take every kind of plan the selection has at that width: the decode
+  stage 1 in 32 splits of 8 key blocks (1 token), stage 1 by sorting in 32
+  splits of 8 blocks (16 tokens) and 16 of 16 (256 tokens), all three reduced
+  and read by pair_decode_read_k16, and stage 1 by thresholds in 2 splits of
+  128 blocks whose stage 2 is fused with the value read (pair_read_k16, 4,096
+  tokens).
 * 268,435,456 fp16 slots (n_sub_keys = 16,384; 137 GB) at 64 tokens, the
   generation workload's per-layer decode batch.
 

@@ -106,7 +106,7 @@ def test_exact_ties_across_flushes(gpu_lib, M, H, n, half, k, score, mode):
     q = torch.tensor(rng.standard_normal((M, H, 2, half)), dtype=torch.float32, device="cuda")
     o = _select(q, _pack(keys, score), n, k, score, mode, torch.full((1,), 10.0, device="cuda"))
     two = _cosines(q, base).topk(2, -1)
-    free = (two.values[..., 0] - two.values[..., 1]) > (2.5 * 2.0 ** -11 if score == F16 else 1e-5)
+    free = (two.values[..., 0] - two.values[..., 1]) > (2.0 ** -9 if score == F16 else 2e-5)  # twice the error below
     assert float(free.float().mean()) > 0.5
     want = torch.tensor(first, dtype=torch.int32, device="cuda")[None].expand(M, -1, -1, -1, -1).gather(
         3, two.indices[..., :1, None].expand(-1, -1, -1, 1, k))[..., 0, :]
@@ -120,8 +120,10 @@ def test_equals_sorted_stage1_and_64_bits(gpu_lib, M, H, n, half, k, score, mode
     """A query's result does not depend on the kernel: every output equals, bit
     for bit, that of calls of few tokens, which take stage 1 by sorting, with
     repeated keys, a NaN key and NaN queries among them.  Other rows against
-    64-bit scores where the k-th and the next are apart by more than the
-    scoring error (a cosine of unit rows rounded to fp16: 2^-11)."""
+    64-bit scores where the k-th and the next are apart by more than twice the
+    scoring error: both rows' components rounded to fp16 move each product by
+    up to 2 * 2^-11 of itself, and sum |q_i k_i| <= 1 for unit rows, so a
+    cosine by 2^-10 (fp32: sums of up to 128 terms, 1e-5)."""
     assert _plan(M, H, n, half, k, score)[0] == _lib.MPL_STAGE1_THRESHOLDS
     g = torch.Generator(device="cuda").manual_seed(n + k)
     q = torch.randn((M, H, 2, half), generator=g, device="cuda")
@@ -133,6 +135,9 @@ def test_equals_sorted_stage1_and_64_bits(gpu_lib, M, H, n, half, k, score, mode
     T = torch.full((1,), 10.0, device="cuda")
     packed = _pack(bad_key, score)
     o = _select(q, packed, n, k, score, mode, T)
+    for _ in range(4):  # and not on the run: its key tiles are overwritten by DMA while the waves go on
+        again = _select(q, packed, n, k, score, mode, T)
+        assert all(torch.equal(a.view(torch.int32), o[name].view(torch.int32)) for name, a in again.items())
     few = next((m for m in (64, 128) if _plan(m, H, n, half, k, score)[0] == _lib.MPL_STAGE1_SORT))
     for r0 in (0, M // 2 + 3, M - few) if few < M else ():
         part = _select(q[r0:r0 + few].contiguous(), packed, n, k, score, mode, T)
@@ -149,13 +154,13 @@ def test_equals_sorted_stage1_and_64_bits(gpu_lib, M, H, n, half, k, score, mode
     cos = _cosines(q[rows], keys)
     cos[:, 1, 0, n // 3] = -2.0
     top = cos.topk(k + 1, -1)
-    err = 2.5 * 2.0 ** -11 if score == F16 else 1e-5
-    free = (top.values[..., k - 1] - top.values[..., k]) > err
-    assert float(free.float().mean()) > 0.1  # k = 32 of 8,192 keys crowd the k-th score
+    err = 2.0 ** -10 if score == F16 else 1e-5
+    free = (top.values[..., k - 1] - top.values[..., k]) > 2 * err
+    assert float(free.float().mean()) > 0.05  # k = 32 of 8,192 keys crowd the k-th score
     got = o["ids"][rows].long()
     assert torch.equal(got[free].sort(-1).values, top.indices[..., :k][free].sort(-1).values)
     scale = 10.0
     if mode == SCALED:
         scale = 10.0 * ((q[rows].double().square().sum(-1, keepdim=True) + 1e-6) / half).sqrt()
     diff = (o["scores"][rows].double() - cos.gather(-1, got.clamp(min=0)) * scale).abs() / scale
-    assert float(diff.max()) < (2.0 ** -11 if score == F16 else 1e-5)
+    assert float(diff.max()) < err

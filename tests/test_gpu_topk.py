@@ -106,14 +106,13 @@ def test_topk_equals_select_stage1(gpu_lib, M, H, n, d_key, k, score, noise):
 
 @pytest.mark.parametrize("M,n", [(16, 8192), (4096, 8192), (16, 16384), (64, 16384)])
 def test_repeated_keys_tie_by_index_across_flushes(gpu_lib, M, n):
-    """Exact ties through the select pass's flushes at the 67M- and 268M-slot
-    key widths (n = 8,192 and 16,384; at 16 and 64 tokens the short splits of
-    4 and 8 blocks): each codebook holds 16 distinct key vectors, each
-    repeated n / 16 times at random places, so a query's best score is
-    reached by that many keys at once and the lane buffers overflow many
-    times.  The top 16 are then the 16 lowest indices holding the best vector
-    (lax.top_k's order, memory.py:34-57), which a flush threshold taken from
-    both lanes of the query must keep: a later key that ties the k-th best
+    """Exact ties at the 67M- and 268M-slot key widths (n = 8,192 and 16,384),
+    through the merges of stage 1 by sorting, which these calls of one head
+    take (test_gpu_thresholds.py has the threshold kernel's flushes): each
+    codebook holds 16 distinct key vectors, each repeated n / 16 times at
+    random places, so a query's best score is reached by that many keys at
+    once, in both lanes of the query and in every split.  The top 16 are then the 16 lowest indices holding the best vector
+    (lax.top_k's order, memory.py:34-57): a later key that ties the k-th best
     loses on its larger index.  Checked on rows whose best and second-best
     distinct vectors are apart by more than the fp16-scoring error."""
     L = _lib.lib()
@@ -166,7 +165,9 @@ def test_stage1_repeats_bit_for_bit(gpu_lib, M, n, noise):
     lands returns a torn vector, a score of no key, which can lift the bound
     above the k-th best and drop candidates, differently from run to run.
     Eight launches on the same inputs at the text-study and 67M-slot key
-    widths, with and without noise, must give identical ids and scores."""
+    widths, with and without noise, must give identical ids and scores.  (The
+    text-study call without noise sorts in registers; at its width the
+    threshold kernel without noise is repeated in test_gpu_thresholds.py.)"""
     L = _lib.lib()
     H, half, k = 4, 128, 16
     g = torch.Generator(device="cuda").manual_seed(n + M + int(noise))
