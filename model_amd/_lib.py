@@ -135,7 +135,7 @@ def stream_ptr(device) -> int:
     (0.2 us of host time against 1.9, on every call into the library)."""
     import torch
 
-    index = getattr(device, "index", None)
-    if index is not None and torch.cuda.is_initialized():
-        return torch._C._cuda_getCurrentRawStream(index)
+    if (type(device) is torch.device and device.index is not None and device.type == "cuda"
+            and torch.cuda.is_initialized()):
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream

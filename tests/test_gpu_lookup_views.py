@@ -61,3 +61,14 @@ def test_both_workspace_places():
     q = torch.randn((96, 4, 64), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
     for M in (4, 96):
         oracle_check(pool, params, q[:M], pool.lookup(params, q[:M]), min_tie_free=0.0)
+
+
+def test_stream_of_any_device_form():
+    """_lib.stream_ptr takes what torch.cuda.current_stream takes, and no other
+    device's stream for a CPU device."""
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for device in ("cuda", "cuda:0", 0, None, torch.device("cuda"), torch.device("cuda", 0)):
+            assert _lib.stream_ptr(device) == side.cuda_stream
+    with pytest.raises(ValueError):
+        _lib.stream_ptr(torch.device("cpu", 0))
