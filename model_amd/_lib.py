@@ -129,13 +129,23 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The CUDA torch.devices with an index that stream_ptr has seen, by index; empty
+# again in a forked child, where torch's own call reports what cannot work.
+_stream_index: dict = {}
+os.register_at_fork(after_in_child=_stream_index.clear)
+
+
 def stream_ptr(device) -> int:
-    """The raw HIP stream that is torch's current one on ``device``.  Asked of
-    the runtime by index where the device has one: no Stream object is made
-    (0.2 us of host time against 1.9, on every call into the library)."""
+    """The raw HIP stream that is torch's current one on ``device`` (what
+    torch.cuda.current_stream takes).  Asked of the runtime by index where the
+    device has one: no Stream object is made (0.2 us of host time against 1.9,
+    on every call into the library)."""
     import torch
 
-    if (type(device) is torch.device and device.index is not None and device.type == "cuda"
-            and torch.cuda.is_initialized()):
-        return torch._C._cuda_getCurrentRawStream(device.index)
-    return torch.cuda.current_stream(device).cuda_stream
+    index = _stream_index.get(device)
+    if index is not None:
+        return torch._C._cuda_getCurrentRawStream(index)
+    stream = torch.cuda.current_stream(device).cuda_stream
+    if type(device) is torch.device and device.index is not None:
+        _stream_index[device] = device.index
+    return stream
