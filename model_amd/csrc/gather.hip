@@ -9,7 +9,7 @@ namespace mpl {
 
 constexpr int kGatherThreads = 256;
 
-template <typename V, int VR, bool NT>
+template <typename V, int VR, bool NT, bool WHOLE>
 __global__ __launch_bounds__(kGatherThreads) void gather_wsum_kernel(
     const V* __restrict__ values, int64_t N, const int32_t* __restrict__ slots,
     const float* __restrict__ weights, int64_t M, int R, int shuffle, float* __restrict__ out) {
@@ -26,8 +26,7 @@ __global__ __launch_bounds__(kGatherThreads) void gather_wsum_kernel(
     if (shuffle) sl = (int)(((int64_t)sl + N / 2 + 1) % N);
     sl = in ? (int)min(max((int64_t)sl, (int64_t)0), N - 1) : 0;  // out-of-range ids read the nearest row
     ww = in ? ww : 0.f;
-    if (R - r0 >= kWave) acc.add_chunk(base, sl, ww, kWave, lane);  // uniform
-    else acc.template add_chunk<true>(base, sl, ww, R - r0, lane);
+    acc.template add_chunk<WHOLE>(base, sl, ww, min(kWave, R - r0), lane);
   }
   acc.store(out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
 }
@@ -83,15 +82,21 @@ static int gather_impl(const V* values, int64_t N, int d, const int32_t* slots, 
     const int VR = (int)(bytes / 16);
     const bool nt = N * bytes > kStreamTableBytes;
     switch (VR) {
-#define MPL_G(vr)                                                                                              \
-  case vr:                                                                                                     \
-    if (nt)                                                                                                    \
-      gather_wsum_kernel<V, vr, true><<<blocks, kGatherThreads, 0, s>>>(values, N, slots, w, M, R, shuffle, out); \
-    else                                                                                                       \
-      gather_wsum_kernel<V, vr, false><<<blocks, kGatherThreads, 0, s>>>(values, N, slots, w, M, R, shuffle, out); \
+#define MPL_GK(vr, NT, WHOLE) \
+  gather_wsum_kernel<V, vr, NT, WHOLE><<<blocks, kGatherThreads, 0, s>>>(values, N, slots, w, M, R, shuffle, out)
+#define MPL_G(vr)                                   \
+  case vr:                                          \
+    if (R % kWave == 0) {                           \
+      if (nt) MPL_GK(vr, true, true);               \
+      else MPL_GK(vr, false, true);                 \
+    } else {                                        \
+      if (nt) MPL_GK(vr, true, false);              \
+      else MPL_GK(vr, false, false);                \
+    }                                               \
     return check_launch("mpl_gather_wsum");
       MPL_G(1) MPL_G(2) MPL_G(4) MPL_G(8) MPL_G(16) MPL_G(32) MPL_G(64) MPL_G(128) MPL_G(256)
 #undef MPL_G
+#undef MPL_GK
       default: break;
     }
     if (VR <= kWave) {

@@ -1182,7 +1182,7 @@ __global__ __launch_bounds__(256) void pair_read_k16(PairParams p, ReadParams rp
   const int64_t N = (int64_t)p.n * p.n;
   if (rp.shuffle) slot = (int)(((int64_t)slot + N / 2 + 1) % N);
   Wsum<V, VR, 16, NT> acc;
-  acc.add_chunk((const uint4*)rp.values, slot, w, 64, lane);
+  acc.template add_chunk<true>((const uint4*)rp.values, slot, w, 64, lane);
   acc.store(rp.out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
 }
 
@@ -1419,7 +1419,7 @@ __global__ __launch_bounds__(1024) void pair_wide_read_k16(PairParams p, ReadPar
     int slot = srow_slot[lane];
     if (rp.shuffle) slot = (int)(((int64_t)slot + N / 2 + 1) % N);
     Wsum<V, VR, 16, NT> sum;
-    sum.add_chunk((const uint4*)rp.values, slot, srow_w[lane], 64, lane);
+    sum.template add_chunk<true>((const uint4*)rp.values, slot, srow_w[lane], 64, lane);
     sum.store(rp.out + m * (int64_t)(VR * Vec16<V>::kElems), lane);
   }
 }

@@ -93,41 +93,56 @@ struct Wsum {
 
   // Adds rows 0..nr-1 of a chunk (nr <= 64): lane i holds row i's slot id
   // `sl` (already in [0, N)) and weight `ww`.  Batches of NB row groups: all
-  // NB loads are issued before any is used.  TAIL: nr < 64, what is loaded for
-  // rows past nr (any row of the table) is zeroed.
-  template <bool TAIL = false>
+  // NB loads are issued before any is used.  WHOLE: nr is 64, whose row groups
+  // are all whole.  Otherwise the loop takes the whole groups, and the rows of
+  // the last one, if it is not, are loaded first and added last, with what the
+  // lanes past nr load (any row of the table) zeroed.
+  template <bool WHOLE>
   __device__ __forceinline__ void add_chunk(const uint4* base, int sl, float ww, int nr, int lane) {
     const int sub = lane / LPR;
     const int col = lane % LPR;
-    const int groups = (nr + RPI - 1) / RPI;
+    const int groups = WHOLE ? kWave / RPI : nr / RPI;
+    const int rest = WHOLE ? 0 : nr % RPI;  // wave-uniform
+    uint4 tail = make_uint4(0, 0, 0, 0);
+    float tw = 0.f;
+    if (rest != 0) {  // never where a row takes the whole wave (RPI = 1)
+      const bool in = sub < rest;
+      const int row = groups * RPI + (in ? sub : 0);
+      const int s = __shfl(sl, row);
+      const float w = __shfl(ww, row);
+      const uint4* src = base + (int64_t)s * VR + col;
+      tail = keep_if(NT ? load_nt(src) : *src, in);
+      tw = in ? w : 0.f;
+    }
     for (int g0 = 0; g0 < groups; g0 += NB) {
       uint4 buf[NB][VPL];
       float wv[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const bool ok = g0 + b < groups;
-        const int row = ok ? (g0 + b) * RPI + sub : 0;  // rows past nr carry weight 0 and slot 0
-        const bool in = ok && row < nr;
-        const int s = __shfl(sl, row);
-        const float w = __shfl(ww, row);
-        wv[b] = ok ? w : 0.f;
-        const uint4* src = base + (int64_t)s * VR + col;
+        if (g0 + b < groups) {  // wave-uniform
+          const int row = (g0 + b) * RPI + sub;
+          const int s = __shfl(sl, row);
+          wv[b] = __shfl(ww, row);
+          const uint4* src = base + (int64_t)s * VR + col;
 #pragma unroll
-        for (int v = 0; v < VPL; ++v) {
-          const uint4 u = NT ? load_nt(src + v * kWave) : src[v * kWave];
-          buf[b][v] = TAIL ? keep_if(u, in) : u;
+          for (int v = 0; v < VPL; ++v) buf[b][v] = NT ? load_nt(src + v * kWave) : src[v * kWave];
         }
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
+        if (g0 + b < groups) {
 #pragma unroll
-        for (int v = 0; v < VPL; ++v) {
-          float f[VE];
-          Vec16<V>::unpack(buf[b][v], f);
+          for (int v = 0; v < VPL; ++v) {
+            float f[VE];
+            Vec16<V>::unpack(buf[b][v], f);
 #pragma unroll
-          for (int e = 0; e < VE; ++e) acc[v][e] = fmaf(wv[b], f[e], acc[v][e]);
+            for (int e = 0; e < VE; ++e) acc[v][e] = fmaf(wv[b], f[e], acc[v][e]);
+          }
         }
       }
+    }
+    if constexpr (VPL == 1) {
+      if (rest != 0) add_vec(tail, tw);
     }
   }
 
@@ -185,33 +200,47 @@ struct WsumAny {
     for (int e = 0; e < VE; ++e) acc[e] = 0.f;
   }
 
-  // Adds rows 0..nr-1 (nr <= 64): lane i holds row i's slot id and weight.
+  // Adds rows 0..nr-1 (nr <= 64): lane i holds row i's slot id and weight;
+  // a last group that is not whole as in Wsum.
   __device__ __forceinline__ void add_chunk(const uint4* base, int sl, float ww, int nr) {
-    for (int r0 = 0; r0 < nr; r0 += NB * RPI) {
+    const int groups = nr / RPI, rest = nr - groups * RPI;  // wave-uniform
+    uint4 tail = make_uint4(0, 0, 0, 0);
+    float tw = 0.f;
+    if (rest != 0) {
+      const bool in = sub < rest;
+      const int row = groups * RPI + (in ? sub : 0);
+      const int s = __shfl(sl, row);
+      const float w = __shfl(ww, row);
+      const uint4* src = base + (int64_t)s * VR + col;
+      tail = keep_if(NT ? load_nt(src) : *src, in);
+      tw = in ? w : 0.f;
+    }
+    for (int g0 = 0; g0 < groups; g0 += NB) {
       uint4 buf[NB];
       float wv[NB];
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const int row = r0 + b * RPI + sub;
-        const bool ok = row < nr;
-        const int s = __shfl(sl, ok ? row : 0);
-        const float w = __shfl(ww, ok ? row : 0);
-        wv[b] = ok && on ? w : 0.f;
-        if (r0 + b * RPI < nr) {  // wave-uniform
+        if (g0 + b < groups) {  // wave-uniform
+          const int row = (g0 + b) * RPI + sub;
+          const int s = __shfl(sl, row);
+          wv[b] = __shfl(ww, row);
           const uint4* src = base + (int64_t)s * VR + col;
-          buf[b] = keep_if(NT ? load_nt(src) : *src, ok);  // lanes past nr read row 0 again
+          buf[b] = NT ? load_nt(src) : *src;
         }
       }
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        if (r0 + b * RPI < nr) {
-          float f[VE];
-          Vec16<V>::unpack(buf[b], f);
-#pragma unroll
-          for (int e = 0; e < VE; ++e) acc[e] = fmaf(wv[b], f[e], acc[e]);
-        }
+        if (g0 + b < groups) add(buf[b], wv[b]);
       }
     }
+    if (rest != 0) add(tail, tw);
+  }
+
+  __device__ __forceinline__ void add(uint4 u, float w) {
+    float f[VE];
+    Vec16<V>::unpack(u, f);
+#pragma unroll
+    for (int e = 0; e < VE; ++e) acc[e] = fmaf(w, f[e], acc[e]);
   }
 
   // Sums the row groups of a column, in a binary tree over sub, and writes

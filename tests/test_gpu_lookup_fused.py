@@ -129,6 +129,8 @@ def test_lookup_zero_tokens_and_errors(gpu_lib):
     (2, 9, 24, torch.float16),    # the read alone, any width
     (2, 9, 256, torch.float16),   # the read alone, 18 rows of a batch of 64
     (1, 5, 128, torch.float32),   # the same, fp32
+    (2, 9, 8, torch.float16),     # one vector a row: all 18 rows in a group of 64
+    (2, 9, 1024, torch.float16),  # two vectors a lane a row
     (8, 10, 512, torch.float16),  # 64 rows and 16 more
 ])
 def test_infinite_entries_stay_infinite(gpu_lib, H, k, d, vdt):
