@@ -128,7 +128,7 @@ int mpl_score_plan(int64_t M, int H, int n, int half, int k, int score_dtype, in
  * outputs as mpl_score_select, plus values [n*n, d] in values_dtype (MPL_F16
  * or MPL_F32), shuffle_reads (memory.py:179) and out [M, d] fp32, which equal
  * mpl_gather_wsum(values, values_dtype, n*n, d, slots, weights, M, H*k,
- * shuffle_reads, out) bit for bit.  With H = 4 and k = 16 the pair stage and
+ * shuffle_reads, out) bit for bit.  With H = 4 and k <= 16 the pair stage and
  * the value read run in one kernel (one wave per token) when the key range is
  * scored in at most 8 splits or reduced to 8 lists.
  */

@@ -35,7 +35,8 @@ FLAGS = [
 
 # Flags of single files, beyond FLAGS.  score_sort.hip: no IEEE mode and no NaN
 # handling of min / max, whose canonicalisation would add an instruction to
-# every key (the file turns NaN scores into -inf before they become keys).
+# every key (the file turns NaN scores into -FLT_MAX, by integer operations on
+# their bits, before they become keys).
 FILE_FLAGS = {"score_sort.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
 
 

@@ -122,9 +122,11 @@ __global__ __launch_bounds__(256, MUL ? 3 : 4) void dense_rows_kernel(DenseArgs 
   const int n0 = (tile - L.tile0) * kTN;
   const int K = p.K;
 
-  // Thread's 16-byte pieces of a chunk: of x, rows tid/16 + 16 i, columns
-  // 4 (tid % 16); of W the same places of a [64][64] block.  Rows and columns
-  // past the ends are read clamped; what lies past K is zeroed in both.
+  // Thread's 16-byte pieces of a chunk of 32 columns of K: of x, rows tid / 8 +
+  // 32 i, columns 4 (tid % 8); of an [N, K] W the same places of a [64][32]
+  // block, of a [K, N] W rows tid / 16 + 16 i, columns 4 (tid % 16) of a
+  // [32][64] block.  Rows and columns past the ends are read clamped; what lies
+  // past K is zeroed in both.
   constexpr int CA = kKC / 4, RA = 256 / CA, NA = kTM / RA;  // row-major operands: columns, rows a pass, passes
   constexpr int NW = LAYOUT == MPL_W_IN_OUT ? kKC / 16 : NA;
   const int pr = tid / CA, pc = 4 * (tid % CA);

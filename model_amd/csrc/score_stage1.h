@@ -23,9 +23,9 @@ struct ScoreParams {
   int64_t M;
   int HC, n, half, k, nblk, splits, blk_per_split;
   int pass1_blocks;  // blocks of each split scanned by the bound pass
-  float* out_sel;    // [splits, HC, k, M] (null without noise: equals clean)
-  float* out_clean;  // [splits, HC, k, M]
-  int* out_idx;      // [splits, HC, k, M]
+  float* out_sel;    // [splits, M, HC, k] (null without noise: equals clean)
+  float* out_clean;  // [splits, M, HC, k]
+  int* out_idx;      // [splits, M, HC, k]
 };
 
 // The wave's MFMA query operand: lane l holds query row my_q (= the wave's

@@ -6,8 +6,9 @@
 // of lax.top_k, ties going to the lowest index.  A double orders by sign and
 // magnitude as a float does, whatever its bits mean, so the score's bits keep
 // their order there; below a negative score the index is stored as it is (a
-// larger magnitude is a smaller key).  No score but a NaN with a payload of
-// all ones makes a double that is not finite, and kNoKey (score -inf, below
+// larger magnitude is a smaller key).  No score makes a double that is not
+// finite but a NaN with the top three bits of its mantissa set (NaN scores
+// become no keys at all: a threshold or a test keeps them out), and kNoKey (score -inf, below
 // every index) marks an empty slot and loses to every real candidate.
 //
 // Why doubles: gfx950 compare-exchanges two of them in registers with one

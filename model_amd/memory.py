@@ -12,7 +12,7 @@ lookup runs in libmpl.so (include/mpl.h) on torch's current HIP stream:
                      + routing softmax
   mpl_gather_wsum    value read                 memory.py:179-193
   mpl_lookup         both of the above in one call (one kernel for
-                     stage 2 and the value read at H = 4, k = 16)
+                     stage 2 and the value read at H = 4, k <= 16)
   mpl_route_counts,  routing statistics, and    memory.py:196-215
   mpl_balance_fwd    the balance loss
   mpl_key_diversity  key_diversity_loss         memory.py:230-240
@@ -40,7 +40,9 @@ NORM_EPS = 1e-6
 # (mpl_lookup_bwd_dense_queries); False keeps the separate query pass.
 FUSED_QUERY_BWD = True
 # Bytes of a lookup's workspace up to which it shares the allocation of the
-# selection lists, which a backward keeps.
+# selection lists (one allocation less, 1 us of host time).  Who keeps the lists
+# (a backward, an aux) then keeps it too: 0.1 MB a token on a large pool, and
+# this at most.
 _WS_WITH_LISTS = 1 << 20
 # In that pass, fp16 operand packs made from the raw queries (normalised in
 # the pack, the same bits as the fp32 q_hat pass); False packs q_hat.
