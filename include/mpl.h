@@ -114,8 +114,10 @@ int mpl_score_select(const void* queries, int query_mode, float* q_len, const vo
  * thresholds), and into how many splits of how many blocks of 32 keys its key
  * range goes (either pointer may be NULL).  noise: with a gumbel tensor; pair:
  * mpl_score_select and mpl_lookup (1) or mpl_score_topk (0).  On the host
- * only; -1 for sizes that those calls refuse.  The choice is a matter of time
- * and never of results.
+ * only; -1 for sizes that those calls refuse.  The choice is a matter of time:
+ * results differ at most in the order of scores that the scaling by the
+ * temperature (and the query's length) rounds to one number, which order by
+ * their unscaled values within a split and as ties between splits.
  */
 enum { MPL_STAGE1_DECODE = 0, MPL_STAGE1_SORT = 1, MPL_STAGE1_THRESHOLDS = 2 };
 int mpl_score_plan(int64_t M, int H, int n, int half, int k, int score_dtype, int noise, int pair, int* splits,

@@ -51,10 +51,18 @@ struct Mfma<_Float16> {
       ss = fmaf(x[i], x[i], ss);
     }
   }
+  // The product rounded to fp32, then to fp16, in every kernel, as the packs of
+  // normalised rows are.  Left to itself the compiler takes v_fma_mixlo_f16,
+  // which rounds once, for some elements of some kernels: one query's operand
+  // then differed by an fp16 step between kernels in one row of some hundreds.  The empty asm keeps the two roundings apart.
   __device__ static Op scale_q(const float* x, float r) {
     Op o;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (_Float16)(x[i] * r);
+    for (int i = 0; i < 8; ++i) {
+      float v = x[i] * r;
+      asm("" : "+v"(v));
+      o[i] = (_Float16)v;
+    }
     return o;
   }
 };

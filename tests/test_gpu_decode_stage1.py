@@ -165,3 +165,29 @@ def test_decode_ties_by_index(gpu_lib, M):
         want = np.nonzero(assign[h, c] == order[m, h, c, 0])[0][:k]
         np.testing.assert_array_equal(ids[m, h, c], want, err_msg=f"row {m} head {h} codebook {c}")
         assert np.all(sc[m, h, c] == sc[m, h, c, 0])
+
+
+@pytest.mark.parametrize("half", [64, 128])
+def test_decode_scores_equal_batched_over_many_rows(gpu_lib, half):
+    """The queries' operand is rounded to fp32 and then to fp16 in every
+    stage-1 kernel.  Rounding once instead differs in one element of 17,000
+    (one row of 128 elements in 130), which some rows of these 1,200 x 8 have."""
+    L = _lib.lib()
+    M, H, n, k = 1200, 4, 256, 4
+    g = torch.Generator(device="cuda").manual_seed(half)
+    q = torch.randn((M, H, 2, half), generator=g, device="cuda")
+    keys = torch.randn((H, 2, n, half), generator=g, device="cuda")
+    st = _lib.stream_ptr(q.device)
+    packed = torch.empty(L.mpl_packed_keys_bytes(H, n, half, _lib.MPL_F16), dtype=torch.uint8, device="cuda")
+    _lib.check(L.mpl_pack_keys(_lib.ptr(keys), H, n, half, _lib.MPL_F16, None, _lib.ptr(packed), st), "pack")
+    T = torch.full((1,), 8.0, device="cuda")
+    ids = torch.full((2, M, H, 2, k), -7, dtype=torch.int32, device="cuda")
+    sc = torch.full((2, M, H, 2, k), 7.0, device="cuda")
+    ws = torch.empty(max(L.mpl_score_topk_workspace_bytes(m, H, n, half, k) for m in (4, M)), dtype=torch.uint8,
+                     device="cuda")
+    for o, m in ((0, M), (1, 4)):
+        for r0 in range(0, M, m):
+            _lib.check(L.mpl_score_topk(q[r0].data_ptr(), _lib.MPL_Q_RAW, None, _lib.ptr(packed), m, H, n, half, k,
+                                        _lib.MPL_F16, _lib.ptr(T), None, None, _lib.ptr(ws), ws.numel(),
+                                        ids[o, r0].data_ptr(), sc[o, r0].data_ptr(), st), "topk")
+    assert torch.equal(ids[0], ids[1]) and torch.equal(sc[0], sc[1])
