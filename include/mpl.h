@@ -81,7 +81,7 @@ int mpl_pack_keys(const float* sub_keys, int H, int n, int half, int score_dtype
  *   query_mode MPL_Q_NORMALIZED: unit rows in score_dtype (fp16 for MPL_F16,
  *     fp32 for MPL_F32, e.g. from mpl_l2_normalize); q_len [M,H,2] is an
  *     input (NULL = no query_scale);
- *   MPL_Q_RAW / MPL_Q_RAW_SCALED (fp16 scoring only): the raw fp32 queries,
+ *   MPL_Q_RAW / MPL_Q_RAW_SCALED: the raw fp32 queries,
  *     l2-normalised inside the kernel (memory.py:30-31, 136); with
  *     MPL_Q_RAW_SCALED the scores are also scaled by
  *     q_len = sqrt(sum q^2 + 1e-6) / sqrt(half), written to q_len if not NULL.

@@ -475,7 +475,7 @@ class MemoryPool:
         staged = None
         if not self.host_pool:
             # selection and value read in one call (memory.py:132-193): with
-            # H = 4 and k = 16 the pair stage and the read share one kernel
+            # H = 4 and k <= 16 the pair stage and the read share one kernel
             values = params["values"]
             if values.dtype not in (torch.float16, torch.float32) or not values.is_contiguous():
                 raise TypeError("values must be a contiguous float16/float32 [n*n, d_value] tensor")

@@ -1,8 +1,8 @@
 """Decode-sized stage 1 (score_topk_decode: at most 4 tokens, fp16 scoring,
-no routing noise) against the batched stage-1 kernel (score_topk_kernel),
-which the other stage-1 tests pin to the oracle: the same queries scored
-alone and as the first rows of an 8-token batch must give the same ids and
-bit-identical scores (the decode kernel runs the batched kernel's MFMA chain
+no routing noise) against the batched stage 1 (by sorting at these sizes,
+score_sort_kernel), which the other stage-1 tests pin to the oracle: the same
+queries scored alone and as the first rows of an 8-token batch must give the
+same ids and bit-identical scores (the decode kernel runs the batched MFMA chain
 with the operands swapped), in every query mode, at ragged key counts,
 padded key widths, k < 16 and the 67M- and 268M-slot key widths.  Also the
 whole lookup at 1-4 tokens (the decode stage 2 and its fused value read:

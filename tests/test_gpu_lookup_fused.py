@@ -1,11 +1,11 @@
 """mpl_lookup (selection and value read in one call) against mpl_score_select
 followed by mpl_gather_wsum, through the C ABI: every output bit for bit.
-Covers the fused stage-2 + read kernel (H = 4, k = 16: fp16 rows of 128, 256
-and 512 elements, fp32 rows, shuffled reads, split-key plans whose lists are
-merged before stage 2), the plans with 9-64 split lists (decode sizes),
-whose lists the fused decode stage 2 (pair_decode_read_k16) reduces, and the
-shapes that fall back to two launches (other H or k, row widths without a
-fused variant)."""
+Covers the fused stage-2 + read kernels (H = 4: k = 16 with fp16 rows of 128,
+256 and 512 elements, fp32 rows, shuffled reads, split-key plans whose lists
+are merged before stage 2; k < 16 and rows of any number of 16-byte vectors up
+to 64), the plans with 9-64 split lists (decode sizes), whose lists the fused
+decode stage 2 (pair_decode_read_k16) reduces, and the shapes that fall back
+to two launches (other H, k > 16, other rows)."""
 
 import pytest
 import torch
@@ -66,8 +66,8 @@ def _run(M, H, n, d_key, d, k, vdt, shuffle, seed):
     (20, 4, 4096, 256, 128, 16, torch.float16, 0),    # 64 split lists
     (9, 4, 2500, 256, 256, 16, torch.float32, 0),     # 40 split lists (ragged n), fp32 rows
     (300, 2, 128, 64, 256, 16, torch.float16, 0),     # H = 2: two launches
-    (300, 4, 128, 64, 256, 8, torch.float16, 0),      # k = 8: two launches
-    (300, 4, 128, 64, 96, 16, torch.float16, 0),      # 96-wide rows: two launches
+    (300, 4, 128, 64, 256, 8, torch.float16, 0),      # k = 8: fused, the rows moved to adjoining lanes
+    (300, 4, 128, 64, 96, 16, torch.float16, 0),      # 96-wide rows: fused, 12 vectors a row
 ])
 def test_lookup_equals_select_then_gather(gpu_lib, M, H, n, d_key, d, k, vdt, shuffle):
     ref, got = _run(M, H, n, d_key, d, k, vdt, shuffle, seed=M + n)

@@ -5,7 +5,7 @@ tests check against the oracle, and against the oracle's top_k directly.
 Ids bit-exact; scores bit-exact to mpl_score_select's (the same kernels and
 the same exact list merges), and within fp16-scoring rounding of the
 oracle's fp64 scores on near-tie-free rows.  Shapes cover one split, split
-lists reduced by merge levels (k = 16) and by the pair kernel (k != 16),
+lists reduced by merge levels (k <= 16) and by the pair kernel (k > 16),
 routing noise, and fp32 scoring, up to the 67M- and 268M-slot key widths
 (n = 8,192 and 16,384) with k = 8, 16 and 32."""
 
@@ -69,7 +69,7 @@ def _run(M, H, n, d_key, k, score, noise, seed):
     (300, 4, 512, 256, 16, _lib.MPL_F16, False),   # text-study keys, one split
     (512, 4, 512, 256, 16, _lib.MPL_F16, False),   # 16 splits: merge levels
     (3, 4, 1024, 256, 16, _lib.MPL_F16, False),    # decode: 32 splits, two levels
-    (37, 2, 64, 16, 4, _lib.MPL_F16, False),       # k != 16 with splits: pair kernel
+    (37, 2, 64, 16, 4, _lib.MPL_F16, False),       # k < 16 with splits
     (5, 2, 640, 32, 16, _lib.MPL_F16, True),       # noise with splits
     (40, 2, 96, 12, 8, _lib.MPL_F32, True),        # fp32 scoring, noise, ragged n
     (256, 4, 8192, 256, 32, _lib.MPL_F16, False),  # k = 32 at the 67M-slot width: split lists, pair kernel
